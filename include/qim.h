@@ -194,16 +194,17 @@ int qim_mxfp8_gemm_ex(const void *aq, const void *as, const void *bq, const void
                       void *out, int64_t ldo, void *out_scales, void *stream);
 
 /* qim_mxfp8_gemm_ex with a caller-provided workspace (no reference
- * counterpart; the same call as optimizations/mxfp8.py:32-36).  When the
- * tile grid's last partial round is a few quarter tiles (at most CUs / 2 of
- * them; e.g. 272 tiles of 256 x 256 on 256 CUs) and the epilogue is
- * QIM_EPI_NONE, QIM_EPI_BIAS or QIM_EPI_GATED_RESIDUAL, each of those quarter
- * tiles is split over K between several workgroups that write fp32 partial
- * sums to ws; a second launch on the same stream adds them in a fixed order
- * and runs the epilogue.  The result is the same function of the inputs
- * within the accumulation order (the partial sums of the tail are added in a
- * different order than one workgroup's MFMA chain).  ws: 16-byte aligned, at
- * least qim_mxfp8_gemm_ws_bytes(M, N, K, epilogue) bytes, not shared by calls
+ * counterpart; the same call as optimizations/mxfp8.py:32-36).  Where a
+ * problem runs 128 x 128 quarter tiles -- a small grid (at most two quarter
+ * tiles per CU), or the last partial round of a grid of 256 x 256 tiles when
+ * that is at most CUs / 2 quarter tiles (e.g. 272 tiles on 256 CUs) -- and the
+ * epilogue is QIM_EPI_NONE, QIM_EPI_BIAS or QIM_EPI_GATED_RESIDUAL, each
+ * quarter tile may be split over K between several workgroups that write fp32
+ * partial sums to ws; a second launch on the same stream adds them in a fixed
+ * order and runs the epilogue.  The result is the same function of the inputs
+ * within the accumulation order (the partial sums are added in a different
+ * order than one workgroup's MFMA chain).  ws: 16-byte aligned, at least
+ * qim_mxfp8_gemm_ws_bytes(M, N, K, epilogue) bytes, not shared by calls
  * that may overlap; with ws = NULL or a smaller ws_bytes the call is
  * qim_mxfp8_gemm_ex. */
 int qim_mxfp8_gemm_ws(const void *aq, const void *as, const void *bq, const void *bs,

@@ -71,12 +71,13 @@ struct GemmArgs {
     // seq / 64 (seq % 64 == 0).
     uint16_t *vt;
     int64_t vt_nkb;
-    // Split-K tail (qim_mxfp8_gemm_ws): with ksplit > 1 each quarter tile of
-    // the last partial round is computed by ksplit workgroups over disjoint
-    // ranges of K, which write their fp32 accumulators to ws; k_mx_gemm_tail
-    // then sums them in a fixed order and runs the epilogue.
+    // Split K (qim_mxfp8_gemm_ws): with ksplit > 1 each quarter tile is computed
+    // by ksplit workgroups over disjoint ranges of K, which write their fp32
+    // accumulators to ws; k_mx_gemm_sum then sums them in a fixed order and
+    // runs the epilogue.
     float *ws;
     int ksplit;
+    int qrows, qcols;  // a grid of quarter tiles only: its rows and columns (qrows 0 otherwise)
 };
 
 // qim_mxfp8_gemm_qk_norm_rope_vt: the QK-norm + RoPE epilogue whose V columns
@@ -504,7 +505,26 @@ __device__ __forceinline__ void epilogue(const GemmArgs &p, f32x16_t (&acc)[TI][
             gpre = *reinterpret_cast<const uint4 *>(p.gate + (int64_t)b0 * p.N + col0 + cl * 8);
         }
         // pass 1
-        if constexpr (SWI) {
+        if constexpr (SWI && TI == 2) {
+            // Quarter tiles compute the SiLU (32 values per lane; filling the
+            // table below would compute as many).
+            static_assert(TJ == 2, "one gate / up tile pair");
+#pragma unroll
+            for (int tl = 0; tl < 2; ++tl) {
+                float g[16], y[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) g[i] = acc[tl][0][i];
+#pragma unroll
+                for (int i = 0; i < 16; i += 2) rbf2(g[i], g[i + 1]);
+                silu_bf16_n<16>(g, y);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) y[i] *= rbf(acc[tl][1][i]);
+#pragma unroll
+                for (int ig = 0; ig < 4; ++ig)
+                    *reinterpret_cast<uint2 *>(reg + (tl * 8 + ig * 2 + kh) * RGS + epi_col_offset<W>(lr)) =
+                        make_uint2(pack_bf16x2(y[4 * ig], y[4 * ig + 1]), pack_bf16x2(y[4 * ig + 2], y[4 * ig + 3]));
+            }
+        } else if constexpr (SWI) {
             // bf16(bf16(silu(g)) * v) for the half's 8 row groups: g and v
             // rounded to bf16 in pairs, every table read of the half issued
             // before the first is used (their latency overlaps the rest), one
@@ -816,15 +836,33 @@ __device__ __forceinline__ void epilogue(const GemmArgs &p, f32x16_t (&acc)[TI][
     }
 }
 
-// ------------------------------------------------------------ tail tiles --
-// The tile grid is rarely a whole number of rounds of the CUs (4352 x 12288:
-// 816 tiles = 3.19 rounds of 256).  The last r tiles (r <= CUs / 2) are then
-// computed as 4r quarter tiles of 128 x 128 by as many extra workgroups, so
-// the last round takes about a quarter of a tile's time instead of a whole
-// one.  A quarter tile: 4 waves in a 2 x 2 grid, each a 64 x 64 block of 2 x 2
-// MFMA tiles, on the same 4-stage LDS ring (half of each operand area used)
-// with the same schedule rules.
-constexpr int QLOADS_EVEN = 5, QLOADS_ODD = 4;  // per wave per stage: 2 A + 2 B (16 B) + 1 scale (4 B, even stages)
+// --------------------------------------------------------- quarter tiles --
+// Quarter tiles of 128 x 128: 4 waves in a 2 x 2 grid, each a 64 x 64 block of
+// 2 x 2 MFMA tiles.  They compute
+//  - the last r tiles (r <= CUs / 2) of a grid of whole tiles (4352 x 12288: 816
+//    tiles = 3.19 rounds of 256), as 4r quarter tiles by as many extra
+//    workgroups of k_mx_gemm, so the last round takes about a quarter of a
+//    tile's time instead of a whole one;
+//  - whole problems whose 256 x 256 tiles would leave most CUs idle
+//    (k_mx_gemm_quarter, gemm_plan).
+// A quarter tile reads twice a whole tile's operand bytes per MFMA from L2 and
+// from LDS, and LDS bounds it: per 128 of K, 33 KiB of DMA writes and 64 KiB of
+// fragment reads against 512 MFMA cycles (measured 0.36 us, ~800 cycles, with the
+// operands in L2; 0.5 us with weights from HBM, where a CU draws 50-70 GB/s
+// however much it has in flight).  So what counts is that its waits overlap: K
+// advances in pairs of 64-byte stages (a pair is one 128-K scale group) with one
+// barrier per pair, each half pair's fragments are read while the other half's
+// MFMAs run, and the pairs go through a ring of NP slots of 33 KiB: NP = 4 where
+// a workgroup has the CU to itself, 2 where two share it (the other's MFMAs then
+// cover its waits).  (Fragments loaded straight into registers, the four waves
+// splitting K and summing their accumulators through LDS at the end, ran the main
+// loop at the MFMA rate from L2 but cost 5.5 us per tile for the exchange: 1280 x
+// 3072 x 3072 19.8 against 16.4 us, x 12288 54.5 against 59 us.)
+constexpr int QTILE_BYTES = 128 * BK;                             // 8 KiB per operand per stage
+constexpr int QSCALE_BYTES = 512;                                 // per operand per pair
+constexpr int QPAIR_BYTES = 4 * QTILE_BYTES + 2 * QSCALE_BYTES;   // A, B of both stages, A and B scales: 33 KiB
+constexpr int QLOADS = 9;  // per wave per pair: 2 x (2 A + 2 B) of 16 B, 1 of 4 B (scales)
+static_assert(4 * QPAIR_BYTES <= LDS_BYTES, "the 4-pair ring fits the whole tile's");
 
 struct QPlan {
     uint32_t a[2], b[2];   // byte offsets into aq / bq (stage 0)
@@ -854,89 +892,127 @@ __device__ __forceinline__ QPlan make_qplan(const GemmArgs &p, int64_t m0, int64
     return Q;
 }
 
-template <bool SCALES>
-__device__ __forceinline__ void issue_qstage(const GemmArgs &p, const QPlan &Q, uint8_t *slot, int s) {
-    const uint32_t ka = (uint32_t)s * Q.astep, kb = (uint32_t)s * Q.bstep, base = lds_addr(slot), w2 = Q.wave * 2;
+// LDS of a pair: stage h (0, 1) has A at h * 16 KiB and B 8 KiB after it; the
+// scales follow both.
+__device__ __forceinline__ void issue_qhalf(const GemmArgs &p, const QPlan &Q, uint8_t *slot, int s) {
+    const uint32_t ka = (uint32_t)s * Q.astep, kb = (uint32_t)s * Q.bstep, w2 = Q.wave * 2;
+    const uint32_t base = lds_addr(slot) + (s & 1) * 2 * QTILE_BYTES;
     dma16(p.aq, Q.a[0] + ka, base + (w2 + 0) * 1024);
     dma16(p.aq, Q.a[1] + ka, base + (w2 + 1) * 1024);
-    dma16(p.bq, Q.b[0] + kb, base + TILE_BYTES + (w2 + 0) * 1024);
-    dma16(p.bq, Q.b[1] + kb, base + TILE_BYTES + (w2 + 1) * 1024);
-    if constexpr (SCALES)
-        dma4(Q.sc_base, Q.sc + (uint32_t)(s >> 1) * 512,
-             base + 2 * TILE_BYTES + (Q.wave < 2 ? 0 : SCALE_BYTES) + (Q.wave & 1) * 256);
+    dma16(p.bq, Q.b[0] + kb, base + QTILE_BYTES + (w2 + 0) * 1024);
+    dma16(p.bq, Q.b[1] + kb, base + QTILE_BYTES + (w2 + 1) * 1024);
+}
+__device__ __forceinline__ void issue_qscales(const QPlan &Q, uint8_t *slot, int t) {
+    dma4(Q.sc_base, Q.sc + (uint32_t)t * 512,
+         lds_addr(slot) + 4 * QTILE_BYTES + (Q.wave < 2 ? 0 : QSCALE_BYTES) + (Q.wave & 1) * 256);
+}
+__device__ __forceinline__ void issue_qpair(const GemmArgs &p, const QPlan &Q, uint8_t *slot, int t) {
+    issue_qhalf(p, Q, slot, 2 * t);
+    issue_qscales(Q, slot, t);
+    issue_qhalf(p, Q, slot, 2 * t + 1);
 }
 
 struct QFrags {
     i32x8_t a[2], b[2];
-    uint2 sa, sb;  // scale dwords of row tiles 0, 1
 };
 
-// Rows h*64 + t*32 + lr (t = 0, 1) of a 128-row scale chunk: dwords at
-// lr*16 + (2h + t)*4, contiguous.
-__device__ __forceinline__ uint2 read_qscales(const uint8_t *base, int h, int lr) {
-    return *reinterpret_cast<const uint2 *>(base + lr * 16 + h * 8);
+// The fragments of half h of a pair, in the order its MFMAs use them.
+__device__ __forceinline__ void read_qfrags(const uint8_t *slot, int h, int wm, int wn, int lr, int kh, QFrags &f) {
+    const uint8_t *A = slot + h * 2 * QTILE_BYTES + 0, *B = A + QTILE_BYTES;
+    f.a[0] = read_tile(A, wm * 64 + lr, kh);
+    f.b[0] = read_tile(B, wn * 64 + lr, kh);
+    f.b[1] = read_tile(B, wn * 64 + 32 + lr, kh);
+    f.a[1] = read_tile(A, wm * 64 + 32 + lr, kh);
 }
 
-__device__ __forceinline__ void read_qfrags(const uint8_t *slot, int wm, int wn, int lr, int kh, QFrags &f, bool scales) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        f.a[t] = read_tile(slot, wm * 64 + t * 32 + lr, kh);
-        f.b[t] = read_tile(slot + TILE_BYTES, wn * 64 + t * 32 + lr, kh);
-    }
-    if (scales) {
-        f.sa = read_qscales(slot + 2 * TILE_BYTES, wm, lr);
-        f.sb = read_qscales(slot + 2 * TILE_BYTES + SCALE_BYTES, wn, lr);
-    }
+// Scale dwords of row tiles 0, 1 of the wave's rows (x, y: A; z, w: B).  Rows
+// h*64 + t*32 + lr (t = 0, 1) of a 128-row scale chunk: dwords at lr*16 + (2h +
+// t)*4, contiguous.
+__device__ __forceinline__ uint4 read_qscales(const uint8_t *slot, int wm, int wn, int lr) {
+    const uint8_t *sc = slot + 4 * QTILE_BYTES;
+    const uint2 a = *reinterpret_cast<const uint2 *>(sc + lr * 16 + wm * 8);
+    const uint2 b = *reinterpret_cast<const uint2 *>(sc + QSCALE_BYTES + lr * 16 + wn * 8);
+    return make_uint4(a.x, a.y, b.x, b.y);
 }
 
-template <int PAR>
-__device__ __forceinline__ void qstep(const GemmArgs &p, const QPlan &Q, uint8_t *lds, int s, int S,
-                                      f32x16_t (&acc)[2][2], const QFrags &cur, QFrags &nxt, int wm, int wn, int lr,
-                                      int kh) {
-    const int sa[2] = {(int)(cur.sa.x >> (8 * kh)), (int)(cur.sa.y >> (8 * kh))};
-    const int sb[2] = {(int)(cur.sb.x >> (8 * kh)), (int)(cur.sb.y >> (8 * kh))};
-#define QIM_QMF(i, j)                                                                                          \
-    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(cur.a[i], cur.b[j], acc[i][j], 0, 0, PAR * 2, \
-                                                                sa[i], PAR * 2, sb[j])
-    QIM_QMF(0, 0);
+// One pair of stages of a quarter tile.  On entry fa holds the even stage's
+// fragments and sc the pair's scales.  First half: the even stage's MFMAs beside
+// the reads of the odd stage.  Then every wave's reads of this slot are done
+// (waited for here) and pair t + 1 has landed for every wave.  Second half: the
+// odd stage's MFMAs beside the reads of pair t + 1 and the issue of pair t + NP
+// into this slot.  REM = 0: inside the K range (pairs t + 1 .. t + NP - 1 are in
+// flight); REM > 0: the REM-th pair from its end, with nothing left to issue and
+// the REM - 1 later pairs in flight.
+template <int NP, int REM>
+__device__ __forceinline__ void qpair_step(const GemmArgs &p, const QPlan &Q, uint8_t *lds, int t, f32x16_t (&acc)[2][2],
+                                           QFrags &fa, uint4 &sc, int wm, int wn, int lr, int kh) {
+    uint8_t *const slot = lds + (t & (NP - 1)) * QPAIR_BYTES;
+    const int sa[2] = {(int)(sc.x >> (8 * kh)), (int)(sc.y >> (8 * kh))};
+    const int sb[2] = {(int)(sc.z >> (8 * kh)), (int)(sc.w >> (8 * kh))};
+    QFrags fb;
+#define QIM_QMF(f, h, i, j)                                                                                        \
+    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.a[i], f.b[j], acc[i][j], 0, 0, (h) * 2, sa[i], \
+                                                                (h) * 2, sb[j])
+    QIM_QMF(fa, 0, 0, 0);
     QIM_SCHED();
-    wait_vmcnt<QLOADS_EVEN + QLOADS_ODD>();
-    block_barrier();
+    read_qfrags(slot, 1, wm, wn, lr, kh, fb);
     QIM_SCHED();
-    issue_qstage<PAR == 0>(p, Q, lds + (s & 3) * STAGE_BYTES, s + 4 < S ? s + 4 : S - 1);
+    QIM_QMF(fa, 0, 0, 1);
+    QIM_QMF(fa, 0, 1, 0);
+    QIM_QMF(fa, 0, 1, 1);
     QIM_SCHED();
-    QIM_QMF(0, 1);
+    if constexpr (REM != 1) {
+        wait_vmcnt<(REM ? REM - 2 : NP - 2) * QLOADS>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        QIM_SCHED();
+    }
+    QIM_QMF(fb, 1, 0, 0);
     QIM_SCHED();
-    if constexpr (PAR == 0) {
-        read_qfrags(lds + ((s + 1) & 3) * STAGE_BYTES, wm, wn, lr, kh, nxt, false);
-        nxt.sa = cur.sa;
-        nxt.sb = cur.sb;
-    } else {
-        read_qfrags(lds + ((s + 1) & 3) * STAGE_BYTES, wm, wn, lr, kh, nxt, true);
+    if constexpr (REM != 1) {
+        const uint8_t *next = lds + ((t + 1) & (NP - 1)) * QPAIR_BYTES;
+        sc = read_qscales(next, wm, wn, lr);
+        read_qfrags(next, 0, wm, wn, lr, kh, fa);
+        QIM_SCHED();
+    }
+    QIM_QMF(fb, 1, 0, 1);
+    QIM_SCHED();
+    if constexpr (REM == 0) issue_qhalf(p, Q, slot, 2 * (t + NP));
+    QIM_SCHED();
+    QIM_QMF(fb, 1, 1, 0);
+    QIM_SCHED();
+    if constexpr (REM == 0) {
+        issue_qscales(Q, slot, t + NP);
+        issue_qhalf(p, Q, slot, 2 * (t + NP) + 1);
     }
     QIM_SCHED();
-    QIM_QMF(1, 0);
-    QIM_QMF(1, 1);
+    QIM_QMF(fb, 1, 1, 1);
     QIM_SCHED();
 #undef QIM_QMF
 }
 
-// fp32 words of one split-K partial: a quarter tile's 4 waves x 2 x 2 MFMA
-// tiles x 16 accumulators x 64 lanes.  Each MFMA tile's 16 accumulators are
-// four groups of 4 (r = 4 g .. 4 g + 3), a group stored as 64 lanes x 16 bytes,
-// so each 16-byte store and load instruction covers 1 KiB contiguous.
-constexpr int QPART_WORDS = 4 * 2 * 2 * 16 * 64;
-
-// Group 0 of the lane's accumulators of MFMA tile (i, j) of a wave; group g
-// is at [64 * g].
-__device__ __forceinline__ float4 *qpart(const GemmArgs &p, int unit, int wave, int i, int j, int lane) {
-    return reinterpret_cast<float4 *>(p.ws + (int64_t)unit * QPART_WORDS) + ((wave * 2 + i) * 2 + j) * 256 + lane;
+// The last min(NP, K range) pairs.
+template <int NP, int REM>
+__device__ __forceinline__ void qtail(const GemmArgs &p, const QPlan &Q, uint8_t *lds, int te, int left,
+                                      f32x16_t (&acc)[2][2], QFrags &fa, uint4 &sc, int wm, int wn, int lr, int kh) {
+    if constexpr (REM > 0) {
+        if (REM <= left) qpair_step<NP, REM>(p, Q, lds, te - REM, acc, fa, sc, wm, wn, lr, kh);
+        qtail<NP, REM - 1>(p, Q, lds, te, left, acc, fa, sc, wm, wn, lr, kh);
+    }
 }
+
+// fp32 words of one split-K partial: a quarter tile, row-major.
+constexpr int QPART_WORDS = 128 * 128;
 
 // Corner of quarter tile q (of the last whole tiles, or a 128-row piece of a
 // last 128-column block).
 __device__ __forceinline__ void quarter_origin(const GemmArgs &p, int q, int64_t &m0, int64_t &n0) {
-    if (q < p.quarters) {  // a quarter of one of the last whole tiles
+    if (p.qrows) {             // a grid of quarter tiles: groups of 8 tile-rows, column-major inside a group
+        const int per_group = 8 * p.qcols, group = q / per_group, first = group * 8;
+        const int gm = p.qrows - first < 8 ? p.qrows - first : 8;
+        const int r = q - group * per_group;
+        m0 = (int64_t)(first + r % gm) * 128;
+        n0 = (int64_t)(r / gm) * 128;
+    } else if (q < p.quarters) {  // a quarter of one of the last whole tiles
         const int tile = p.main_tiles + q / 4, quarter = q & 3;
         int tm, tn;
         tile_coords(p, tile, tm, tn);
@@ -948,12 +1024,11 @@ __device__ __forceinline__ void quarter_origin(const GemmArgs &p, int q, int64_t
     }
 }
 
-// Quarter-tile unit u: quarter tile u % quarters over K-stage pairs
+// Quarter-tile unit u: quarter tile u % quarters over the stage pairs
 // [kp * P / ksplit, (kp + 1) * P / ksplit), kp = u / quarters, P = K / 128 (the
-// whole of K when ksplit == 1).  Stages keep their ring slot (s & 3) and
-// their parity (even stages carry the 128-K scale group).
-template <int EPI>
-__device__ __forceinline__ void quarter_tile(const GemmArgs &p, uint8_t *lds, uint8_t *tab, int u) {
+// whole of K when ksplit == 1).
+template <int EPI, int NP>
+__device__ __forceinline__ void quarter_tile(const GemmArgs &p, uint8_t *lds, int u) {
     const int split = p.ksplit > 1 ? p.ksplit : 1;
     const int q = split > 1 ? u % p.quarters : u, kp = split > 1 ? u / p.quarters : 0;
     int64_t m0, n0;
@@ -962,43 +1037,44 @@ __device__ __forceinline__ void quarter_tile(const GemmArgs &p, uint8_t *lds, ui
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, kh = lane >> 5;
     const int P = (int)(p.K / (2 * BK));
-    const int sb = 2 * (kp * P / split), se = 2 * ((kp + 1) * P / split);
+    const int tb = kp * P / split, te = (kp + 1) * P / split;
     f32x16_t acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = f32x16_t{};
     const QPlan Q = make_qplan(p, m0, n0);
-    issue_qstage<true>(p, Q, lds + (sb & 3) * STAGE_BYTES, sb);
-    issue_qstage<false>(p, Q, lds + ((sb + 1) & 3) * STAGE_BYTES, sb + 1);
-    issue_qstage<true>(p, Q, lds + ((sb + 2) & 3) * STAGE_BYTES, sb + 2 < se ? sb + 2 : se - 1);
-    issue_qstage<false>(p, Q, lds + ((sb + 3) & 3) * STAGE_BYTES, sb + 3 < se ? sb + 3 : se - 1);
-    if constexpr (ring_offset<EPI>() > 0) fill_silu_table(tab);
-    wait_vmcnt<QLOADS_ODD + QLOADS_EVEN + QLOADS_ODD>();  // stage sb landed
+    const int left = te - tb < NP ? te - tb : NP;  // pairs of the prologue (ksplit <= P: at least one)
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+        if (i < left) issue_qpair(p, Q, lds + ((tb + i) & (NP - 1)) * QPAIR_BYTES, tb + i);
+    // Pair tb landed: the left - 1 pairs after it may be in flight.
+    if (left == NP)
+        wait_vmcnt<(NP - 1) * QLOADS>();
+    else
+        wait_vmcnt<0>();
     block_barrier();
-    QFrags fa, fb;
-    read_qfrags(lds + (sb & 3) * STAGE_BYTES, wm, wn, lr, kh, fa, true);
-    for (int s = sb; s < se; s += 2) {
-        qstep<0>(p, Q, lds, s, se, acc, fa, fb, wm, wn, lr, kh);
-        qstep<1>(p, Q, lds, s + 1, se, acc, fb, fa, wm, wn, lr, kh);
-    }
-    wait_vmcnt<0>();
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (split > 1) {  // a partial sum: to the workspace, the epilogue runs in k_mx_gemm_tail
+    QFrags fa;
+    const uint8_t *first = lds + (tb & (NP - 1)) * QPAIR_BYTES;
+    uint4 sc = read_qscales(first, wm, wn, lr);
+    read_qfrags(first, 0, wm, wn, lr, kh, fa);
+    for (int t = tb; t < te - NP; ++t) qpair_step<NP, 0>(p, Q, lds, t, acc, fa, sc, wm, wn, lr, kh);
+    qtail<NP, NP>(p, Q, lds, te, left, acc, fa, sc, wm, wn, lr, kh);
+    if (split > 1) {  // a partial sum: to the workspace, the epilogue runs in k_mx_gemm_sum
+        float *w = p.ws + (int64_t)u * QPART_WORDS + (wm * 64 + 4 * kh) * 128 + wn * 64 + lr;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i) {
+            if (m0 + wm * 64 + i * 32 >= p.M) break;  // rows nobody reads
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                float4 *w = qpart(p, u, wave, i, j, lane);
+            for (int r = 0; r < 16; ++r)
 #pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    w[64 * g] = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
-                                            acc[i][j][4 * g + 3]);
-            }
+                for (int j = 0; j < 2; ++j) w[(32 * i + 8 * (r / 4) + r % 4) * 128 + 32 * j] = acc[i][j][r];
+        }
         return;
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     block_barrier();
-    epilogue<EPI, 2, 2>(p, acc, lds, tab, m0 + wm * 64, n0 + wn * 64, lane, wave);
+    epilogue<EPI, 2, 2>(p, acc, lds, nullptr, m0 + wm * 64, n0 + wn * 64, lane, wave);
 }
 
 template <int EPI>
@@ -1008,7 +1084,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // (and the epilogue's staging) follows it.
     uint8_t *const tab = smem, *const lds = smem + ring_offset<EPI>();
     if ((int)blockIdx.x >= p.main_tiles) {  // a quarter tile of the last partial round
-        quarter_tile<EPI>(p, lds, tab, (int)blockIdx.x - p.main_tiles);
+        quarter_tile<EPI, 4>(p, lds, (int)blockIdx.x - p.main_tiles);
         return;
     }
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1048,64 +1124,81 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     epilogue<EPI, 4, 4>(p, acc, lds, tab, m0 + wm * 128, n0 + wn * 128, lane, wave);
 }
 
-// The split-K tail's second launch: one one-wave workgroup per 64 x 64 block
-// of a quarter tile (workgroup 4 q + w does wave w's block of quarter q) sums
-// its ksplit partials in order kp = 0, 1, ... (the register layout the
-// quarter tile's wave wrote, each partial's 16 loads in flight together) and
-// runs that block's epilogue.  At 64 quarter tiles x 4 splits this takes
-// 6.8 us, against 7.8 us with one four-wave workgroup per quarter tile.
-constexpr int TAIL_LDS_BYTES = 16 * (64 * 8 + 8 * 16);  // epilogue<EPI, 2, 2>'s staging of one wave (TJ = 2, bf16 rows)
+// A grid of quarter tiles only (gemm_plan): NP = 4 while the units are no more
+// than the CUs; else NP = 2, two per CU.
+constexpr int qlds_bytes(int np) { return np * QPAIR_BYTES; }
 
+template <int EPI, int NP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mx_gemm_quarter(GemmArgs p) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    // Contiguous ranges of units per XCD (workgroup ids go round-robin over 8).
+    const int n = gridDim.x, xcd = blockIdx.x & 7, base = n >> 3, rem = n & 7;
+    quarter_tile<EPI, NP>(p, smem, xcd * base + (xcd < rem ? xcd : rem) + (int)(blockIdx.x >> 3));
+}
+
+// The split-K second launch: sums each quarter tile's ksplit partials in order
+// kp = 0, 1, ... and runs the plain, bias or gated-residual epilogue.  One
+// lane per 8 columns of a row (16 lanes per row of a quarter, 16 rows per
+// workgroup), so that a few rows still spread over many waves; a lane's loads of
+// four partials are in flight together.
 template <int EPI>
-__global__ __launch_bounds__(64) void k_mx_gemm_tail(GemmArgs p) {
-    static_assert(ring_offset<EPI>() == 0, "the split tail runs the plain, bias and gated-residual epilogues");
-    __shared__ __attribute__((aligned(16))) uint8_t lds[TAIL_LDS_BYTES];
-    const int q = (int)(blockIdx.x >> 2);
+__global__ __launch_bounds__(256) void k_mx_gemm_sum(GemmArgs p) {
+    static_assert(ring_offset<EPI>() == 0, "the split runs the plain, bias and gated-residual epilogues");
+    const int q = (int)blockIdx.x, r = (int)blockIdx.y * 16 + (threadIdx.x >> 4), c = (threadIdx.x & 15) * 8;
     int64_t m0, n0;
     quarter_origin(p, q, m0, n0);
-    if (m0 >= p.Mp) return;
-    const int lane = threadIdx.x, wave = (int)(blockIdx.x & 3);
-    const int wm = wave >> 1, wn = wave & 1;
-    f32x16_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const float4 *w = qpart(p, q, wave, i, j, lane);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 v = w[64 * g];
-                acc[i][j][4 * g] = v.x;
-                acc[i][j][4 * g + 1] = v.y;
-                acc[i][j][4 * g + 2] = v.z;
-                acc[i][j][4 * g + 3] = v.w;
-            }
-        }
-    for (int kp = 1; kp < p.ksplit; ++kp) {
-        // all 16 loads of a partial in flight before its adds
-        const int u = kp * p.quarters + q;
-        float4 v[2][2][4];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const float4 *w = qpart(p, u, wave, i, j, lane);
-#pragma unroll
-                for (int g = 0; g < 4; ++g) v[i][j][g] = w[64 * g];
-            }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    acc[i][j][4 * g] += v[i][j][g].x;
-                    acc[i][j][4 * g + 1] += v[i][j][g].y;
-                    acc[i][j][4 * g + 2] += v[i][j][g].z;
-                    acc[i][j][4 * g + 3] += v[i][j][g].w;
-                }
+    const int64_t row = m0 + r, col = n0 + c;
+    if (row >= p.M) return;
+    [[maybe_unused]] uint4 hv, gv;
+    if constexpr (EPI == QIM_EPI_GATED_RESIDUAL) {
+        hv = ld_nt(p.res + row * p.N + col);
+        gv = *reinterpret_cast<const uint4 *>(p.gate + ((uint32_t)row / (uint32_t)p.seq) * p.N + col);
+    } else if constexpr (EPI == QIM_EPI_BIAS) {
+        gv = *reinterpret_cast<const uint4 *>(p.bias + col);
     }
-    epilogue<EPI, 2, 2>(p, acc, lds, nullptr, m0 + wm * 64, n0 + wn * 64, lane, 0);  // LDS region 0: its own
+    const float4 *w = reinterpret_cast<const float4 *>(p.ws + (int64_t)q * QPART_WORDS + r * 128 + c);
+    const int64_t step = (int64_t)p.quarters * (QPART_WORDS / 4);
+    float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int kp = 0; kp < p.ksplit; kp += 4) {
+        float4 a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (kp + i < p.ksplit) {
+                a[i] = w[(kp + i) * step];
+                b[i] = w[(kp + i) * step + 1];
+            } else {
+                a[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            y[0] += a[i].x; y[1] += a[i].y; y[2] += a[i].z; y[3] += a[i].w;
+            y[4] += b[i].x; y[5] += b[i].y; y[6] += b[i].z; y[7] += b[i].w;
+        }
+    }
+    const int64_t o = row * p.ldo + col;
+    if constexpr (EPI == EPI_F32) {
+        float *out = reinterpret_cast<float *>(p.out) + o;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) out[t] = y[t];
+    } else if constexpr (EPI == EPI_F16) {
+        _Float16 *out = reinterpret_cast<_Float16 *>(p.out) + o;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) out[t] = (_Float16)y[t];
+    } else {
+        if constexpr (EPI == QIM_EPI_BIAS) {
+            float bv[8];
+            unpack8(gv, bv);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) y[t] += bv[t];
+        } else if constexpr (EPI == QIM_EPI_GATED_RESIDUAL) {
+            float h[8], g[8];
+            unpack8(hv, h);
+            unpack8(gv, g);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) y[t] = h[t] + rbf(g[t] * rbf(y[t]));
+        }
+        st_nt(reinterpret_cast<uint16_t *>(p.out) + o, pack8(y));
+    }
 }
 
 // CUs the work split plans for: the current device's, or MI355X's 256 when no
@@ -1124,37 +1217,97 @@ static int64_t main_tile_count(int64_t tiles) {
     return (r > 0 && 2 * r <= cus) ? tiles - r : tiles;
 }
 
+template <int EPI, int NP>
+static int launch_quarters(const GemmArgs &a, int64_t units, hipStream_t st) {
+    static std::atomic<bool> configured[QIM_MAX_DEVICES] = {};
+    if (const int rc = reserve_lds(reinterpret_cast<const void *>(&k_mx_gemm_quarter<EPI, NP>), qlds_bytes(NP), configured,
+                                   "qim_mxfp8_gemm"))
+        return rc;
+    launch(k_mx_gemm_quarter<EPI, NP>, dim3((unsigned)units), dim3(256), qlds_bytes(NP), st, a);
+    return QIM_OK;
+}
+
 template <int EPI>
 static int launch_gemm(const GemmArgs &a, hipStream_t st) {
     static std::atomic<bool> configured[QIM_MAX_DEVICES] = {};
-    constexpr int lds_bytes = LDS_BYTES + ring_offset<EPI>();
-    if (const int rc = reserve_lds(reinterpret_cast<const void *>(&k_mx_gemm<EPI>), lds_bytes, configured,
-                                   "qim_mxfp8_gemm"))
-        return rc;
-    const int64_t half_column = a.tiles_n * BN < a.N ? (a.Mp + 127) / 128 : 0;
     const int64_t split = a.ksplit > 1 ? a.ksplit : 1;
-    const int64_t grid = a.main_tiles + a.quarters * split + half_column;
-    launch(k_mx_gemm<EPI>, dim3((unsigned)grid), dim3(256), lds_bytes, st, a);
-    if constexpr (ring_offset<EPI>() == 0 && EPI != QIM_EPI_QK_NORM_ROPE && EPI != EPI_QKV_VT) {
-        if (split > 1) launch(k_mx_gemm_tail<EPI>, dim3((unsigned)a.quarters * 4), dim3(64), 0, st, a);
+    if (a.qrows) {
+        const int64_t units = a.quarters * split;
+        if (const int rc = units <= plan_cus() ? launch_quarters<EPI, 4>(a, units, st) : launch_quarters<EPI, 2>(a, units, st))
+            return rc;
+    } else {
+        constexpr int lds_bytes = LDS_BYTES + ring_offset<EPI>();
+        if (const int rc = reserve_lds(reinterpret_cast<const void *>(&k_mx_gemm<EPI>), lds_bytes, configured,
+                                       "qim_mxfp8_gemm"))
+            return rc;
+        const int64_t half_column = a.tiles_n * BN < a.N ? (a.Mp + 127) / 128 : 0;
+        const int64_t grid = a.main_tiles + a.quarters * split + half_column;
+        launch(k_mx_gemm<EPI>, dim3((unsigned)grid), dim3(256), lds_bytes, st, a);
+    }
+    if constexpr (ring_offset<EPI>() == 0 && !is_qk_epi<EPI>()) {
+        if (split > 1) launch(k_mx_gemm_sum<EPI>, dim3((unsigned)a.quarters, 8), dim3(256), 0, st, a);
     }
     return QIM_OK;
 }
 
-// K-splits of the tail's quarter tiles: as many as fill the CUs' one round
-// (quarters * ksplit <= CUs), at most one stage pair each and at most 8; 1
-// (no split) when the quarters alone hold more than half the CUs, when a last
-// 128-column block is there, or for an epilogue other than the plain, bias
-// and gated-residual ones.
-static int tail_ksplit(int64_t quarters, bool half_column, int epilogue, int64_t K) {
-    const int64_t cus = plan_cus();
-    if (quarters <= 0 || half_column) return 1;
-    if (epilogue != QIM_EPI_NONE && epilogue != QIM_EPI_BIAS && epilogue != QIM_EPI_GATED_RESIDUAL) return 1;
-    int64_t k = cus / quarters;
-    const int64_t pairs = K / (2 * BK);
-    if (k > pairs) k = pairs;
-    if (k > 8) k = 8;
-    return k >= 2 ? (int)k : 1;
+static bool splits_k(int epilogue) {
+    return epilogue == QIM_EPI_NONE || epilogue == QIM_EPI_BIAS || epilogue == QIM_EPI_GATED_RESIDUAL;
+}
+
+// How one problem runs: main_tiles whole tiles, then the quarter tiles of the
+// other whole tiles (times ksplit) and those of a last 128-column block; or,
+// with qrows set, quarters = qrows x qcols quarter tiles only (times ksplit).
+struct GemmPlan {
+    int64_t main_tiles, quarters, qrows, qcols;
+    int ksplit;
+    int64_t ws_bytes() const { return ksplit > 1 ? quarters * ksplit * (int64_t)QPART_WORDS * 4 : 0; }
+};
+
+// K-splits of a grid of quarter tiles, from a cost model in microseconds fitted
+// to sweeps over M 40..512 (weights cold, each time best of the splits within 10 %):
+// 0.5 per stage pair (a CU draws ~66 GB/s of operands while few CUs run), 5
+// for the summing launch, and the partials' traffic (32-row groups below M,
+// written and read) at 5 TB/s.  40 x 3072 x 12288: 48.7 us unsplit, 15.5 us in 8;
+// 512 x 4096 x 4096: 17.6 us unsplit, 19.9 us in 2 (kept unsplit).
+static int quarter_ksplit(int64_t quarters, int64_t M, int64_t N, int64_t pairs) {
+    const double partial = (double)((M + 31) / 32 * 32) * (double)N * 8.0 / 5e6;
+    double best = 0.5 * (double)pairs;
+    int64_t ksplit = 1;
+    for (int64_t k = 2; k <= 8 && k <= pairs && k * quarters <= plan_cus(); ++k) {
+        const double cost = 0.5 * (double)((pairs + k - 1) / k) + 5.0 + (double)k * partial;
+        if (cost < best) {
+            best = cost;
+            ksplit = k;
+        }
+    }
+    return (int)ksplit;
+}
+
+static GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int epilogue) {
+    const int64_t cus = plan_cus(), pairs = K / (2 * BK);
+    const int64_t Mp = (M + 127) / 128 * 128, tiles_n = N / BN, tiles = (Mp + BM - 1) / BM * tiles_n;
+    const int64_t qrows = Mp / 128, qcols = N / 128;
+    // Quarter tiles only, when all of them fit the chip at once, two per CU: at
+    // most half as many whole tiles as CUs would run.  1280 x 3072 x 3072 (60 whole
+    // tiles) 28.3 -> 15.0 us, x 12288 104.7 -> 59 us; 2048 x 4096 x 4096 (128)
+    // 38.5 -> 32.6 us; 1024 x 9216 x 3072 (144) 32.6 -> 35.9 us (kept whole).
+    if (qrows * qcols <= 2 * cus) {
+        const int64_t q = qrows * qcols;
+        return GemmPlan{0, q, qrows, qcols, splits_k(epilogue) ? quarter_ksplit(q, M, N, pairs) : 1};
+    }
+    const int64_t main = main_tile_count(tiles);
+    GemmPlan pl{main, 4 * (tiles - main), 0, 0, 1};
+    // K-splits of the tail's quarter tiles: as many as fill the CUs' one round
+    // (quarters * ksplit <= CUs), at most one stage pair each and at most 8; 1
+    // (no split) when the quarters alone hold more than half the CUs, when a last
+    // 128-column block is there, or for an epilogue other than the plain, bias
+    // and gated-residual ones.
+    if (pl.quarters > 0 && tiles_n * BN == N && splits_k(epilogue)) {
+        int64_t k = cus / pl.quarters;
+        k = k < pairs ? k : pairs;
+        pl.ksplit = (int)(k > 8 ? 8 : k >= 2 ? k : 1);
+    }
+    return pl;
 }
 
 }  // namespace qim
@@ -1168,14 +1321,6 @@ struct QKNormRope {
     int64_t heads;
     void *vt;  // V^T tiles instead of the V columns of out, or null
 };
-
-// Quarter tiles and K-splits of the tail for a problem shape (tail_ksplit).
-static void tail_plan(int64_t M, int64_t N, int64_t K, int epilogue, int64_t &quarters, int &ksplit) {
-    const int64_t Mp = (M + 127) / 128 * 128, tiles_m = (Mp + BM - 1) / BM, tiles_n = N / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    quarters = 4 * (tiles - main_tile_count(tiles));
-    ksplit = tail_ksplit(quarters, tiles_n * BN < N, epilogue, K);
-}
 
 static int gemm_run(const void *aq, const void *as, const void *bq, const void *bs, int64_t M, int64_t N, int64_t K,
                     int epilogue, int layouts, const void *bias, const void *gate, const void *res, int64_t seq,
@@ -1224,17 +1369,16 @@ static int gemm_run(const void *aq, const void *as, const void *bq, const void *
         a.vt = static_cast<uint16_t *>(qk->vt);
         a.vt_nkb = seq / 64;
     }
-    const int64_t tiles = tiles_m * tiles_n;
-    a.main_tiles = (int)main_tile_count(tiles);
-    a.quarters = (int)(4 * (tiles - a.main_tiles));
-    if (ws && !qk) {
-        int64_t quarters;
-        int ksplit;
-        tail_plan(M, N, K, epilogue, quarters, ksplit);
+    const GemmPlan pl = gemm_plan(M, N, K, epilogue);
+    a.main_tiles = (int)pl.main_tiles;
+    a.quarters = (int)pl.quarters;
+    a.qrows = (int)pl.qrows;
+    a.qcols = (int)pl.qcols;
+    if (ws) {
         QIM_REQUIRE(aligned16(ws), QIM_ERR_LAYOUT, "qim_mxfp8_gemm_ws: ws must be 16-byte aligned");
-        if (ksplit > 1 && ws_bytes >= quarters * ksplit * (int64_t)QPART_WORDS * 4) {
+        if (pl.ksplit > 1 && ws_bytes >= pl.ws_bytes()) {
             a.ws = static_cast<float *>(ws);
-            a.ksplit = ksplit;
+            a.ksplit = pl.ksplit;
         }
     }
     int rc;
@@ -1297,10 +1441,7 @@ extern "C" int qim_mxfp8_gemm_ex(const void *aq, const void *as, const void *bq,
 
 extern "C" int64_t qim_mxfp8_gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int epilogue) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128 || N % 128) return 0;
-    int64_t quarters;
-    int ksplit;
-    tail_plan(M, N, K, epilogue, quarters, ksplit);
-    return ksplit > 1 ? quarters * ksplit * (int64_t)QPART_WORDS * 4 : 0;
+    return gemm_plan(M, N, K, epilogue).ws_bytes();
 }
 
 extern "C" int qim_mxfp8_gemm_ws(const void *aq, const void *as, const void *bq, const void *bs, int64_t M,

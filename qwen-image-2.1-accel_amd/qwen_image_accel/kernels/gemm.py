@@ -140,9 +140,9 @@ def mx_matmul(activation, weight_fp8, weight_scale, *, epilogue="none", bias=Non
     args = (_native.ptr(a.values), _native.ptr(a.scales), _native.ptr(w), _native.ptr(weight_scale), m, n, k, epi,
             layouts, _native.ptr(bias), _native.ptr(gate), _native.ptr(residual), int(seq or m), _native.ptr(buf),
             ldo, _native.ptr(out_scales))
-    # A tile grid whose last partial round is a few quarter tiles splits them
-    # over K with a workspace from torch's caching allocator (stream-ordered,
-    # so reusing it for the next call on the stream is safe).
+    # A small grid, or one whose last partial round is a few quarter tiles,
+    # splits them over K with a workspace from torch's caching allocator
+    # (stream-ordered, so reusing it for the next call on the stream is safe).
     ws_bytes = _native.lib().qim_mxfp8_gemm_ws_bytes(m, n, k, epi) if epi in _WS_EPILOGUES else 0
     if ws_bytes > 0:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)

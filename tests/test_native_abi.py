@@ -166,6 +166,28 @@ def test_gemm_workspace_bytes():
     assert lib.qim_mxfp8_gemm_ws_bytes(0, 4096, 4096, none) == 0
 
 
+def test_gemm_workspace_bytes_quarter_grids():
+    """Grids of quarter tiles only (at most two per CU) split K for the same
+    epilogues while the units fit one round of the CUs, at most 8 ways and one
+    stage pair each, and only where the summing launch costs less than it saves."""
+    lib = _native.lib()
+    part, none, swq = 64 * 1024, _native.EPI_NONE, _native.EPI_SWIGLU_QUANT
+    for m in (1, 40, 128, 129, 512, 1280, 2048):
+        for n in (128, 384, 3072, 4096, 9216):
+            quarters = (m + 127) // 128 * (n // 128)
+            if quarters > 512:
+                continue
+            for k in (128, 256, 1152, 4096, 12288):
+                got = lib.qim_mxfp8_gemm_ws_bytes(m, n, k, none)
+                ksplit, rest = divmod(got, quarters * part)
+                assert rest == 0 and ksplit != 1
+                assert ksplit <= min(8, k // 128) and ksplit * quarters <= 256
+                assert lib.qim_mxfp8_gemm_ws_bytes(m, n, k, swq) == 0
+    assert lib.qim_mxfp8_gemm_ws_bytes(40, 3072, 12288, none) == 24 * 8 * part
+    assert lib.qim_mxfp8_gemm_ws_bytes(512, 4096, 4096, none) == 0   # the partials' traffic outweighs the split
+    assert lib.qim_mxfp8_gemm_ws_bytes(1280, 3072, 12288, none) == 0  # 240 quarters fill the CUs
+
+
 def test_attention_workspace_bytes():
     """V^T tiles (16 KiB per batch, head and 64-key block), plus, when the last
     partial round of work items is split over key ranges (the work split only

@@ -12,17 +12,27 @@
 // query, exchange one value per block.  An S^T accumulator is already the B
 // operand of the P V product: lane (q, h = l / 32) holds keys
 // {8(i/4) + 4h + i%4}, i = 0..15, of its 32-key tile, so values 0-7 are its 8
-// keys of the first 16-key MFMA step and 8-15 of the second.  V^T is stored
-// with each 16-key group in that order ([0-3, 8-11 | 4-7, 12-15]), so the A
-// operand of lane (d, h) is one contiguous 16-byte read.  (An MFMA pairs the
-// K slots of A and B by position, so any key order works as long as A and B
-// agree.)
+// keys of the first 16-key MFMA step and 8-15 of the second.  The A operand of
+// lane (d, h) is the same 8 keys of V's column d.  (An MFMA pairs the K slots of A
+// and B by position, so any key order works as long as A and B agree.)
 //
-// V^T comes from a transpose pass (k_attn_vt) into a workspace: one 16 KiB
-// tile per (batch, head, 64-key block), 128 rows (d) of 64 keys, with the
-// 16-byte chunk c of row d at chunk c ^ ((d >> 1) & 7) (conflict-free reads of
-// 16 lanes with consecutive d).  K is loaded straight from the K tensor, with
-// chunk c of key r at chunk c ^ (r & 15) in LDS.
+// V comes in one of two forms.  Rows: loaded straight from the V tensor and
+// transposed by the LDS reads (two ds_read_b64_tr_b16 of 4 keys per operand).  V^T
+// tiles: written to the workspace by the QKV GEMM's epilogue, or by a transpose
+// pass (k_attn_vt) where the queries are many (ATT_VROWS_MAX_S): one 16 KiB tile
+// per (batch, head, 64-key block), 128 rows (d) of 64 keys with each 16-key group
+// in the operand order ([0-3, 8-11 | 4-7, 12-15]), so that an operand is one
+// 16-byte read, and the 16-byte chunk c of row d at chunk c ^ ((d >> 1) & 7)
+// (conflict-free reads of 16 lanes with consecutive d).  K is loaded straight from
+// the K tensor, with chunk c of key r at chunk c ^ (r & 15) in LDS.
+//
+// What bounds it: long runs draw the power limit (S = T = 16640, 24 heads: ~1.74
+// GHz, the matrix cores busy 71 % of the waves' cycles, 47.7 cycles per 32-cycle
+// MFMA; 58 with the row sums on v_dot2c_f32_bf16, 54 as the compiler scheduled
+// them).  S 16640 2950 -> 2850 us, S 4096 x T 8392 (32 heads) 588 -> 536 us, S 1024
+// x T 1101 (2 x 32 heads) 62 -> 44 us including the transpose pass this drops.
+#include <type_traits>
+
 #include "qim_attention.h"
 #include "qim_device.h"
 #include "qim_runtime.h"
@@ -31,20 +41,21 @@ namespace qim {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16a_t __attribute__((ext_vector_type(16)));
+typedef float f32x4a_t __attribute__((ext_vector_type(4)));
 
 constexpr int ATT_D = 128;          // head dim
 constexpr int ATT_KB = 64;          // keys per block
 constexpr int ATT_BQ = 256;         // queries per workgroup: 4 waves x 2 tiles of 32
 constexpr int ATT_TILE = ATT_KB * ATT_D * 2;  // 16 KiB: one K block or one V^T block
-constexpr int ATT_STAGE = 2 * ATT_TILE;       // K + V^T
 constexpr int ATT_NSTAGE = 4;
-constexpr int ATT_LDS = ATT_NSTAGE * ATT_STAGE;  // 128 KiB
+constexpr int ATT_LDS = ATT_NSTAGE * 2 * ATT_TILE;  // 128 KiB
 
 struct AttnArgs {
     const uint16_t *q, *k;
-    const uint16_t *vt;  // V^T tiles
+    const uint16_t *vt;  // V^T tiles (k_attn_fwd<., true>)
+    const uint16_t *v;   // V rows (k_attn_fwd<., false>)
     uint16_t *o;
-    int64_t ldq, ldk, ldo;  // elements between consecutive tokens
+    int64_t ldq, ldk, ldv, ldo;  // elements between consecutive tokens
     int S, T, H, nkb;       // queries, keys, heads, key blocks
     int nq;                 // query blocks per (batch, head)
     // Work split (att_plan): workgroups [0, nfull) each run one whole work item
@@ -62,6 +73,7 @@ struct AttnArgs {
     uint8_t *qcodes, *qscales;
     int64_t Mp;
     int tiled;
+    int o_vec16;  // rows of o are 16-byte aligned
 };
 
 // One query row's 4-column group of an MXFP8 output: code byte offset.
@@ -106,109 +118,171 @@ __global__ __launch_bounds__(256) void k_attn_vt(const uint16_t *__restrict__ v,
 }
 
 // ------------------------------------------------------------- forward --
-__device__ __forceinline__ void att_dma16(const void *base, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"(lds_addr)
-                 : "memory");
-}
-__device__ __forceinline__ uint32_t att_lds_addr(const void *p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
-}
 template <int N>
 __device__ __forceinline__ void att_wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-__device__ __forceinline__ bf16x8_t as_bf16x8(const uint4 &u) { return __builtin_bit_cast(bf16x8_t, u); }
+// LDS: a ring of 4 K blocks (16 KiB each), then a ring of 4 V blocks.  Block n
+// is in slot gray(n % 4) (0, 1, 3, 2), so going to the next block flips one
+// address bit: 14 after even blocks, 15 after odd ones.
+constexpr int ATT_VRING = ATT_NSTAGE * ATT_TILE;
+__device__ __forceinline__ uint32_t att_flip(int n) { return (uint32_t)ATT_TILE << (n & 1); }
+typedef __attribute__((address_space(3))) const u32x4_t *att_lds_vec_t;
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
 // DMA addressing of one wave's share of a key block: 4 instructions of K and
-// 4 of V^T (1 KiB each).  K instruction j (n = 4 wave + j) covers keys
-// 4n..4n+3 of the block: lane i lands at LDS row r = 4n + i/16, physical chunk
-// i % 16, whose source is the key's logical chunk (i % 16) ^ (r & 15).  Per
-// block only the (wave-uniform) base address moves; the per-lane offsets are
-// fixed, with a second set for the last block whose rows past T - 1 are
-// clamped to T - 1 (their scores are masked).  V^T tiles are copied as they are.
+// 4 of V (1 KiB each).  Instruction j (n = 4 wave + j) covers keys 4n..4n+3 of
+// the block: lane i lands at LDS row r = 4n + i/16, physical chunk i % 16, whose
+// source is the row's logical chunk (i % 16) ^ (r & 15) for K and
+// (i % 16) ^ 4 (r & 3) for V rows; V^T tiles are copied as they are.  An
+// instruction's offset field moves its LDS and its global address alike, so the
+// four share one M0; the per-lane offsets are reduced by 1 KiB j and raised by
+// ATT_BIAS, which the base pointers are lowered by.  Per block only the
+// (wave-uniform) bases move; before the last block its rows past T - 1 are
+// clamped to T - 1 (their scores are masked; V rows are zeroed in LDS).
+constexpr int ATT_BIAS = 3072;
 struct AttLoader {
-    const uint8_t *k0;            // K row 0 of this (batch, head)
-    const uint8_t *vt0;           // V^T tile 0 of this (batch, head)
-    int64_t kstep;                // bytes of K per key block
-    uint32_t koff[4], klast[4];   // per-lane K offsets: full blocks, the last block
-    uint32_t voff;                // per-lane V^T offset
-    int lastb;
+    const uint8_t *kp, *vp;    // K and V of the next block to issue
+    int64_t kstep, vstep;      // bytes per block
+    uint32_t koff[4], voff[4]; // per-lane offsets (voff[0] only for V^T tiles)
+    uint32_t lds;              // LDS address of this wave's share of the next slot
+    int next, last;            // the next block and the range's last one
+    int rmax;                  // last valid row of the range's last block (>= 63: whole)
 };
 
-__device__ __forceinline__ AttLoader att_loader(const AttnArgs &p, int b, int h, int wave, int lane) {
-    AttLoader L;
-    L.k0 = reinterpret_cast<const uint8_t *>(p.k + (int64_t)b * p.T * p.ldk + (int64_t)h * ATT_D);
-    L.vt0 = reinterpret_cast<const uint8_t *>(p.vt + ((int64_t)b * p.H + h) * p.nkb * (ATT_KB * ATT_D));
-    L.kstep = (int64_t)ATT_KB * p.ldk * 2;
-    L.lastb = p.nkb - 1;
-    const int rmax = p.T - 1 - L.lastb * ATT_KB;  // last valid row of the last block
+template <bool VT>
+__device__ __forceinline__ void att_offsets(const AttnArgs &p, AttLoader &L, int wave, int lane, int rmax) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int r = 4 * (wave * 4 + j) + (lane >> 4);
-        const int c = (lane & 15) ^ (r & 15);
-        const int rl = r < rmax ? r : rmax;
-        L.koff[j] = (uint32_t)(((int64_t)r * p.ldk + c * 8) * 2);
-        L.klast[j] = (uint32_t)(((int64_t)rl * p.ldk + c * 8) * 2);
+        const int r = 4 * (wave * 4 + j) + (lane >> 4), rl = r < rmax ? r : rmax;
+        const int adj = ATT_BIAS - 1024 * j;
+        L.koff[j] = (uint32_t)(((int64_t)rl * p.ldk + ((lane & 15) ^ (r & 15)) * 8) * 2 + adj);
+        L.voff[j] = VT ? (uint32_t)(wave * 4096 + lane * 16 + ATT_BIAS)
+                       : (uint32_t)(((int64_t)rl * p.ldv + ((lane & 15) ^ ((r & 3) << 2)) * 8) * 2 + adj);
     }
-    L.voff = (uint32_t)(wave * 4096 + lane * 16);
+}
+
+// A wave-uniform pointer in scalar registers (the DMA's base operand).
+__device__ __forceinline__ const uint8_t *att_uniform(const uint8_t *ptr) {
+    const uint64_t a = reinterpret_cast<uint64_t>(ptr);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return reinterpret_cast<const uint8_t *>((uint64_t)hi << 32 | lo);
+}
+
+template <bool VT>
+__device__ __forceinline__ AttLoader att_loader(const AttnArgs &p, int b, int h, int kb0, int nkb, int wave, int lane) {
+    AttLoader L;
+    L.kstep = (int64_t)ATT_KB * p.ldk * 2;
+    L.vstep = VT ? ATT_TILE : (int64_t)ATT_KB * p.ldv * 2;
+    L.kp = reinterpret_cast<const uint8_t *>(p.k + (int64_t)b * p.T * p.ldk + (int64_t)h * ATT_D) + kb0 * L.kstep - ATT_BIAS;
+    L.vp = (VT ? reinterpret_cast<const uint8_t *>(p.vt + ((int64_t)b * p.H + h) * p.nkb * (ATT_KB * ATT_D))
+               : reinterpret_cast<const uint8_t *>(p.v + (int64_t)b * p.T * p.ldv + (int64_t)h * ATT_D)) +
+           kb0 * L.vstep - ATT_BIAS;
+    L.kp = att_uniform(L.kp);
+    L.vp = att_uniform(L.vp);
+    L.lds = wave * 4096;
+    L.next = 0;
+    L.last = nkb - 1;
+    L.rmax = p.T - 1 - (kb0 + nkb - 1) * ATT_KB;
+    att_offsets<VT>(p, L, wave, lane, ATT_KB);
     return L;
 }
 
-// Issue key block kb (clamped by the caller to the last block) into an LDS slot.
-__device__ __forceinline__ void att_issue(const AttLoader &L, int wave, uint8_t *slot, int kb) {
-    const uint32_t base = att_lds_addr(slot) + wave * 4096;
-    const uint8_t *kp = L.k0 + kb * L.kstep;
-    if (kb == L.lastb) {
+template <int OFF>
+__device__ __forceinline__ void att_dma16(const uint8_t *base, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(voff), "s"(base), "{m0}"(lds_addr), "n"(OFF)
+                 : "memory");
+}
+
+// Before a block's DMA: the clamped offsets of a last block that is not whole.
+template <bool VT>
+__device__ __forceinline__ void att_issue_begin(const AttnArgs &p, AttLoader &L, int wave, int lane) {
+    if (L.next == L.last && L.rmax < ATT_KB - 1) att_offsets<VT>(p, L, wave, lane, L.rmax);
+}
+// DMA instruction `part` of the next block (0-3: K, 4-7: V).
+template <bool VT>
+__device__ __forceinline__ void att_issue_part(const AttLoader &L, int part) {
+    const uint32_t k = L.lds, v = L.lds + ATT_VRING;
+    if (part == 0) att_dma16<0>(L.kp, L.koff[0], k);
+    if (part == 1) att_dma16<1024>(L.kp, L.koff[1], k);
+    if (part == 2) att_dma16<2048>(L.kp, L.koff[2], k);
+    if (part == 3) att_dma16<3072>(L.kp, L.koff[3], k);
+    if (part == 4) att_dma16<0>(L.vp, L.voff[0], v);
+    if (part == 5) att_dma16<1024>(L.vp, VT ? L.voff[0] : L.voff[1], v);
+    if (part == 6) att_dma16<2048>(L.vp, VT ? L.voff[0] : L.voff[2], v);
+    if (part == 7) att_dma16<3072>(L.vp, VT ? L.voff[0] : L.voff[3], v);
+}
+// After it: on to the next block (the last one again past the end, into a slot
+// that is never read).
+__device__ __forceinline__ void att_issue_end(AttLoader &L, uint32_t flip) {
+    const bool more = L.next < L.last;
+    L.kp += more ? L.kstep : 0;
+    L.vp += more ? L.vstep : 0;
+    L.next += more ? 1 : 0;
+    L.lds ^= flip;
+}
+
+// LDS addresses of a lane's fragments in the current slots (the kernel's LDS
+// starts at address 0); sub-blocks and V's head-dim tiles (V^T) or key steps (V
+// rows) are offsets of the reads themselves.
+//   K, head-dim step j: lane (r = key % 32, hf) reads d [16j + 8hf, +8) of key r.
+//   V^T, 16-key step kk of the block: lane (d % 32, hf) reads the 8 keys that
+//     pair with its P^T operand; head dims 32 dt + d % 32.
+//   V rows, head-dim tile dt: the transposing read gives lane i of a 16-lane
+//     group column i of the 4 x 16 block whose row j is held by lanes 4j..4j+3,
+//     so lane l addresses 8 bytes of key 4hf + (l % 16) / 4 (and 8 keys later),
+//     d 32 dt + 16 ((l / 16) % 2) + 4 (l % 4); the chunk swizzle 4 (key % 4)
+//     spreads the 4 keys over all banks.
+struct AttAddr {
+    uint32_t k[8], v[4];
+};
+template <bool VT>
+__device__ __forceinline__ AttAddr att_addr(int lane) {
+    AttAddr A;
+    const int lq = lane & 31, hf = lane >> 5, i = lane & 15;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) att_dma16(kp, L.klast[j], base + j * 1024);
+    for (int j = 0; j < 8; ++j) A.k[j] = lq * 256 + (((2 * j + hf) ^ (lq & 15)) << 4);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        A.v[t] = ATT_VRING +
+                 (VT ? lq * (ATT_KB * 2) + (((2 * t + hf) ^ ((lq >> 1) & 7)) << 4)
+                     : (4 * hf + (i >> 2)) * 256 + ((t ^ (i >> 2)) << 6) + ((lane >> 4) & 1) * 32 + (i & 3) * 8);
+    return A;
+}
+__device__ __forceinline__ bf16x8_t att_read_k(const AttAddr &A, int j, int off) {
+    return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<att_lds_vec_t>((uintptr_t)(A.k[j] + off)));
+}
+// V fragment of 16-key step kk, head-dim tile dt.
+template <bool VT>
+__device__ __forceinline__ bf16x8_t att_read_v(const AttAddr &A, int kk, int dt) {
+    if constexpr (VT) {
+        return __builtin_bit_cast(bf16x8_t,
+                                  *reinterpret_cast<att_lds_vec_t>((uintptr_t)(A.v[kk] + dt * (32 * ATT_KB * 2))));
     } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) att_dma16(kp, L.koff[j], base + j * 1024);
+        typedef __attribute__((address_space(3))) i16x4_t *ptr_t;
+        const uint32_t at = A.v[dt] + kk * (16 * ATT_D * 2);
+        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<ptr_t>((uintptr_t)at));
+        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<ptr_t>((uintptr_t)(at + 8 * ATT_D * 2)));
+        return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
-    const uint8_t *tile = L.vt0 + (int64_t)kb * ATT_TILE;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) att_dma16(tile, L.voff + j * 1024, base + ATT_TILE + j * 1024);
 }
 
-// K fragments of one 32-key sub-block (half hb of an LDS key block), all 8
-// head-dim steps: lane (r = key % 32, hf) reads d [16j + 8hf, +8) of key r.
-__device__ __forceinline__ void att_read_k(uint4 (&kf)[8], const uint8_t *kt_lds, int hb, int lq, int hf) {
-    const int r = 32 * hb + lq;
+// The loader of a range, its first three blocks issued.
+template <bool VT>
+__device__ __forceinline__ AttLoader att_start(const AttnArgs &p, int b, int h, int kb0, int nkb, int wave, int lane) {
+    AttLoader ld = att_loader<VT>(p, b, h, kb0, nkb, wave, lane);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        kf[j] = *reinterpret_cast<const uint4 *>(kt_lds + r * 256 + (((2 * j + hf) ^ (r & 15)) * 16));
+    for (int i = 0; i < 3; ++i) {
+        att_issue_begin<VT>(p, ld, wave, lane);
+#pragma unroll
+        for (int part = 0; part < 8; ++part) att_issue_part<VT>(ld, part);
+        att_issue_end(ld, att_flip(i));
+    }
+    return ld;
 }
 
-// V^T fragments of one 32-key sub-block: lane (d % 32, hf) reads the 8 keys of
-// 16-key step kk = 2hb + u that pair with its P^T operand, head dims 32dt + d % 32.
-__device__ __forceinline__ void att_read_v(uint4 (&vf)[2][4], const uint8_t *vt_lds, int hb, int lq, int hf) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            const int d = 32 * dt + lq, kk = 2 * hb + u;
-            vf[u][dt] = *reinterpret_cast<const uint4 *>(vt_lds + d * (ATT_KB * 2) + (((2 * kk + hf) ^ ((d >> 1) & 7)) * 16));
-        }
-}
-
-// S^T of one 32-query tile over one 32-key sub-block: 8 MFMAs.
-__device__ __forceinline__ void att_scores(f32x16a_t &s, const uint4 (&kf)[8], const uint4 (&qf)[8]) {
-    s = f32x16a_t{};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[j]), as_bf16x8(qf[j]), s, 0, 0, 0);
-}
-
-// O^T += V^T P^T for one 32-query tile over one 32-key sub-block: 8 MFMAs.
-__device__ __forceinline__ void att_pv(f32x16a_t (&o)[4], const uint4 (&vf)[2][4], const uint4 (&pf)[2]) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vf[u][dt]), as_bf16x8(pf[u]), o[dt], 0, 0, 0);
-}
-
-// Keys at or past T (the partial last sub-block) get a score of -inf.
+// Keys at or past T (the partial last block) get a score of -inf.
 __device__ __forceinline__ void att_mask(f32x16a_t &s, int kbase, int T, int hf) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -218,38 +292,6 @@ __device__ __forceinline__ void att_mask(f32x16a_t &s, int kbase, int T, int hf)
 }
 
 __device__ __forceinline__ float att_max(float a, float b) { return __builtin_elementwise_maximum(a, b); }
-
-// Keep a softmax inside the region whose MFMAs it runs beside: the compiler
-// would otherwise sink it past the branch that ends the region.
-__device__ __forceinline__ void att_pin(uint4 (&pf)[2], float &x) {
-    u32x4_t v0 = {pf[0].x, pf[0].y, pf[0].z, pf[0].w}, v1 = {pf[1].x, pf[1].y, pf[1].z, pf[1].w};
-    asm volatile("" : "+v"(v0), "+v"(v1), "+v"(x));
-    pf[0] = make_uint4(v0.x, v0.y, v0.z, v0.w);
-    pf[1] = make_uint4(v1.x, v1.y, v1.z, v1.w);
-}
-
-// P = 2^(s c - m) for this lane's 16 keys of query lq, written as the bf16 B
-// operands of the P V product; returns their sum (of the bf16 values used).
-__device__ __forceinline__ float att_exp_pack(const f32x16a_t &s, float m, uint4 (&pf)[2], float c) {
-    const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
-    float sum0 = 0.f, sum1 = 0.f;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        uint32_t w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * u + 2 * e], c, -m));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * u + 2 * e + 1], c, -m));
-            w[e] = pack_bf16x2(p0, p1);
-        }
-        pf[u] = make_uint4(w[0], w[1], w[2], w[3]);
-        sum0 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w[0]), ones, sum0, false);
-        sum1 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w[1]), ones, sum1, false);
-        sum0 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w[2]), ones, sum0, false);
-        sum1 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w[3]), ones, sum1, false);
-    }
-    return sum0 + sum1;
-}
 
 // The (unscaled) row max of a score tile over both half-waves (the other
 // half-wave holds the other 16 keys of the same query).
@@ -265,186 +307,251 @@ __device__ __forceinline__ float att_rowmax(const f32x16a_t &s) {
     return att_max(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
 }
 
+// One 32-query tile of a wave: scores, P^T operands, O^T and the statistics.
+// P of 16 keys x 32 queries per MFMA step: w[0..3] and w[4..7], packed bf16.
+struct AttTile {
+    f32x16a_t s, o[4];
+    uint32_t w[8];
+    float e[2];     // P of a pair not yet packed
+    float m;        // reference max (log2 units)
+    f32x4a_t l;     // this lane's sum of P (of the bf16 values used), in every element
+};
+__device__ __forceinline__ bf16x8_t att_p(const AttTile &t, int u) {
+    const u32x4_t v = {t.w[4 * u], t.w[4 * u + 1], t.w[4 * u + 2], t.w[4 * u + 3]};
+    return __builtin_bit_cast(bf16x8_t, v);
+}
+
+// P = 2^(s c - m) of score k of a tile (called for k = 0..17 in order): the
+// exponential of score k, and for even k the packing of the pair before it (one
+// slot later, so that nothing waits for an exponential).  One slot after every
+// second pair its and the previous pair's four values are added to l: v_mfma_f32_4x4x4_16b_bf16 with an
+// all-ones A is, for each lane, the sum of the lane's own four B values.  (As
+// v_dot2c_f32_bf16, eight per 16 scores, the sums slowed the MFMAs beside them:
+// 49.4 against 37.4 cycles per MFMA without them, loads left out.)
+__device__ __forceinline__ void att_exp(AttTile &t, int k, float c, i16x4_t ones) {
+    if (k > 0 && k <= 16 && (k & 1) == 0) {
+        uint32_t w = pack_bf16x2(t.e[0], t.e[1]);
+        // Keeps the work in its slot: it would otherwise sink to where P is used.
+        asm volatile("" : "+v"(w));
+        t.w[k / 2 - 1] = w;
+    }
+    if (k > 4 && (k & 3) == 1) {
+        const u32x2_t v = {t.w[(k - 1) / 2 - 2], t.w[(k - 1) / 2 - 1]};
+        t.l = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(i16x4_t, v), t.l, 0, 0, 0);
+    }
+    if (k < 16) t.e[k & 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(t.s[k], c, -t.m));
+}
+
 // Online softmax with a running max (the safe form).  Scores above the
 // reference max m by at most ATT_RESCALE (log2 units) are exponentiated
 // against m as they are (P <= 2^ATT_RESCALE); a sub-block whose max exceeds
-// that moves m to its max.  Updates m and the partial sum l (this lane's keys;
-// the half-waves' sums are added at the end) and returns the factor O must be
-// multiplied by before this sub-block's P V.
+// that moves m to its max and rescales l and O (skipped, wave-uniform, when no
+// query of the wave moved its max).
 constexpr float ATT_RESCALE = 8.0f;
 
-__device__ __forceinline__ float att_softmax(const f32x16a_t &s, float &m, float &l, uint4 (&pf)[2], float c) {
-    const float mx = att_rowmax(s) * c;
-    const float mnew = mx > m + ATT_RESCALE ? mx : m;
-    float alpha = __builtin_amdgcn_exp2f(m - mnew);  // 1 if m stays, 0 on the first sub-block
-    m = mnew;
-    l = l * alpha + att_exp_pack(s, mnew, pf, c);
-    att_pin(pf, alpha);
-    return alpha;
-}
-
-// o *= alpha, skipped (wave-uniform) when no query of the wave moved its max.
-__device__ __forceinline__ void att_rescale(f32x16a_t (&o)[4], float alpha) {
+__device__ __forceinline__ void att_softmax_safe(AttTile &t, float c, i16x4_t ones) {
+    const float mx = att_rowmax(t.s) * c;
+    const float mnew = mx > t.m + ATT_RESCALE ? mx : t.m;
+    const float alpha = __builtin_amdgcn_exp2f(t.m - mnew);  // 1 if m stays, 0 on the first sub-block
+    t.m = mnew;
+    t.l *= alpha;
+#pragma unroll
+    for (int k = 0; k <= 17; ++k) att_exp(t, k, c, ones);
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+        for (int dt = 0; dt < 4; ++dt) t.o[dt] *= alpha;
     }
 }
 
-// The softmax of one region.  FIXED: against the reference max m fixed by
-// the tile's first sub-block (no max, no rescale: l += sum, nothing to branch
-// on); otherwise the safe form above.  att_sm_end runs at the region's end,
-// after its LDS reads are issued.
-template <bool FIXED>
-__device__ __forceinline__ float att_sm(const f32x16a_t &s, float &m, float &l, uint4 (&pf)[2], float c) {
-    if constexpr (FIXED) {
-        float sum = att_exp_pack(s, m, pf, c);
-        att_pin(pf, sum);
-        return sum;
-    } else {
-        return att_softmax(s, m, l, pf, c);
-    }
-}
-template <bool FIXED>
-__device__ __forceinline__ void att_sm_end(f32x16a_t (&o)[4], float &l, float r) {
-    if constexpr (FIXED) l += r;
-    else att_rescale(o, r);
+#define ATT_SCHED() __builtin_amdgcn_sched_barrier(0)
+
+// Waits until at most N of this wave's LDS reads are outstanding.  A builtin,
+// not assembly: the compiler sees it and adds no wait per fragment (each a
+// 4-cycle instruction) after it.
+template <int N>
+__device__ __forceinline__ void att_wait_lds() {
+    static_assert(N <= 15, "lgkmcnt is 4 bits");
+    __builtin_amdgcn_s_waitcnt(0xC07F | (N << 8));
 }
 
-// One pass over all keys for this wave's 64 queries: two 32-query tiles
-// (0, 1), keys in 32-key sub-blocks u (two per 64-key LDS block).  Per
-// sub-block the work is S_t = K Q_t^T, the softmax SM_t and O_t += V^T P_t^T;
-// it runs software-pipelined in two steps so that each softmax runs on the
-// vector ALU beside 16 MFMAs that do not depend on it:
-//   X(u): MFMA S_1(u), PV_1(u-1)   | VALU SM_0(u) | LDS reads of V^T(u), K(u+1)
-//   Y(u): MFMA PV_0(u), S_0(u+1)   | VALU SM_1(u)
-// Every K and V^T fragment is read from LDS once and used for both query
-// tiles; the fragments alternate between two register sets by the parity of u.
-// LDS holds four 64-key blocks: block n + 2 is issued into the slot of block
-// n - 2 at the barrier before X(2n - 1), after the last read of that slot.
+// One region: 16 MFMAs of tile A -- its scores with the K fragments `kf`, then
+// O += V^T P^T with the V fragments `vf` -- beside the softmax of tile B, in 16
+// slots of one MFMA and one score each.  A lone wave issues at most one
+// instruction per 4.4 cycles (5.4 for an 8-byte one, 8.5 for an exponential), so
+// a slot of one MFMA, a score's fma and exponential, half a pack and a row sum and
+// one LDS read just fits the MFMA's 32 cycles.  (Left to itself the compiler
+// bunched the softmax into the first half of each region, left the rest to bare
+// MFMAs, and waited for each fragment separately.)  `work(k)` is the slot's memory
+// work.  LDSK: the fragments were read in the previous region, K first; at most
+// LDSK reads (V's) may be outstanding at the first score, none at the first P V.
+// FAST: B's reference max is fixed, nothing to rescale; otherwise the safe
+// softmax runs whole, before the MFMAs.
+template <bool FAST, bool SCORES, bool PV, bool SOFTMAX, int LDSK, class F>
+__device__ __forceinline__ void att_region(AttTile &A, AttTile &B, const bf16x8_t (&q)[8], const bf16x8_t (&kf)[8],
+                                           bf16x8_t (&vf)[2][4], float c, i16x4_t ones, F &&work) {
+    if constexpr (!FAST && SOFTMAX) att_softmax_safe(B, c, ones);
+    if constexpr (LDSK >= 0 && SCORES) att_wait_lds<LDSK>();
+    if (FAST) ATT_SCHED();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        if (k < 8) {
+            if constexpr (SCORES)
+                A.s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[k], q[k], k == 0 ? f32x16a_t{} : A.s, 0, 0, 0);
+        } else {
+            if constexpr (PV) {
+                const int u = (k - 8) / 4, dt = k & 3;
+                A.o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u][dt], att_p(A, u), A.o[dt], 0, 0, 0);
+            }
+        }
+        if (FAST) ATT_SCHED();
+        if constexpr (FAST && SOFTMAX) att_exp(B, k, c, ones);
+        work(k);
+        if (LDSK >= 0 && PV && k == 7) {
+            att_wait_lds<0>();
+            // V fragments live in accumulation registers (MFMA operands only):
+            // the architectural ones hold O, the scores and P.
+#pragma unroll
+            for (int i = 0; i < 8; ++i) asm volatile("" : "+a"(vf[i / 4][i & 3]));
+        }
+        if (FAST) ATT_SCHED();
+    }
+    if constexpr (FAST && SOFTMAX) {
+        att_exp(B, 16, c, ones);
+        att_exp(B, 17, c, ones);
+    }
+    if (FAST) ATT_SCHED();
+}
+
+// One pass over the key blocks of a range for this wave's 64 queries: two
+// 32-query tiles (0, 1), keys in 32-key sub-blocks u (two per 64-key LDS
+// block).  Per sub-block the work is S_t = K Q_t^T, the softmax SM_t and O_t +=
+// V^T P_t^T; it runs software-pipelined in two regions so that each softmax
+// runs on the vector ALU beside 16 MFMAs that do not depend on it:
+//   Y(u): MFMA S_0(u + 1), PV_0(u)   | VALU SM_1(u) | DMA of block n + 3
+//   X(u): MFMA S_1(u), PV_1(u - 1)   | VALU SM_0(u) | LDS reads of K(u + 1), V(u)
+// Every K and V fragment is read from LDS once and used for both query tiles;
+// its successor is read right after its last use (in X), 8 to 16 MFMAs before
+// the successor's first (in Y).  Block n + 3 is issued into the ring slot of
+// block n - 1 after the barrier before X(2n + 1), which follows the last read of
+// that slot.
 //
 // FAST: after each tile's first sub-block (which sets m to its max) the
 // reference max stays fixed, so a region has no max, no rescale and no branch.
 // P may then exceed 1 by the growth of the scores past the first sub-block's
 // max; the caller checks that l stayed below ATT_FAST_LMAX (so that P, l and O
 // stayed finite) and otherwise reruns the pass with FAST = false.
-template <bool FAST>
-__device__ __forceinline__ void att_pass(const AttnArgs &p, const AttLoader &ld, uint8_t *lds, const uint4 (&qf)[2][8],
-                                         int wave, int lq, int hf, int kb0, int nkb, f32x16a_t (&o0)[4],
-                                         f32x16a_t (&o1)[4], float &m0, float &m1, float &l0, float &l1) {
+template <bool FAST, bool VT>
+__device__ __forceinline__ void att_pass(const AttnArgs &p, AttLoader ld, uint8_t *lds, const bf16x8_t (&qf)[2][8],
+                                         int wave, int lane, int kb0, int nkb, AttTile &t0, AttTile &t1) {
     // Key blocks [kb0, kb0 + nkb); n below counts from kb0.  Keys past T exist
     // only in the last block of T; a sub-block there may be all masked, which
     // gives P = 0 and leaves m, l and O as they are.
-    const int lastb = nkb - 1;
-    const bool ragged = kb0 + nkb == p.nkb && (p.T & (ATT_KB - 1)) != 0;
-    const int key0 = kb0 * ATT_KB;
+    const int hf = lane >> 5, lastb = nkb - 1;
+    const int kl = (kb0 + lastb) * ATT_KB;  // first key of the last block
+    const bool ragged = p.T - kl < ATT_KB;
     const float c = p.scale_log2e;
+    const i16x4_t ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};  // bf16 1.0
+    AttAddr A = att_addr<VT>(lane);
+    bf16x8_t kf[8], vf[2][4];
+    t0.m = t1.m = -__builtin_inff();
+    t0.l = t1.l = f32x4a_t{};
 #pragma unroll
-    for (int i = 0; i < 3; ++i) att_issue(ld, wave, lds + i * ATT_STAGE, kb0 + (i < nkb ? i : lastb));
+    for (int dt = 0; dt < 4; ++dt) t0.o[dt] = t1.o[dt] = f32x16a_t{};
 
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) o0[dt] = o1[dt] = f32x16a_t{};
-    m0 = m1 = -__builtin_inff();
-    l0 = l1 = 0.f;
-    uint4 kfa[8], kfb[8], vfa[2][4], vfb[2][4], pf0[2], pf1[2];
-    f32x16a_t s0, s1;
-    auto slot = [&](int n) { return lds + (n & 3) * ATT_STAGE; };
-
-    // Block 0 landed for every wave.  S_0(0); X(0) without a P V, whose
-    // softmax (the safe form) sets tile 0's reference max; in a FAST pass
-    // tile 1's is set here from S_1(0) as well.
+    // V rows past the last key count as zeros (V^T tiles hold zeros there).
+    auto zero_rows = [&](int slot) {
+        if (VT) return;
+        const int tail = p.T - kl;
+        for (int i = threadIdx.x; i < (ATT_KB - tail) * 16; i += 256)
+            *reinterpret_cast<uint4 *>(lds + ATT_VRING + slot * ATT_TILE + tail * 256 + i * 16) = make_uint4(0, 0, 0, 0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    // Block 0 landed for every wave: S_0(0), S_1(0), SM_0(0), which sets the
+    // tiles' reference max.
     att_wait_vmcnt<16>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    att_read_k(kfa, lds, 0, lq, hf);
-    att_scores(s0, kfa, qf[0]);
-    if (lastb == 0 && ragged) att_mask(s0, key0, p.T, hf);
-    {
-        att_scores(s1, kfa, qf[1]);
-        const float r = att_sm<false>(s0, m0, l0, pf0, c);
-        att_read_v(vfa, slot(0) + ATT_TILE, 0, lq, hf);
-        att_read_k(kfb, slot(0), 1, lq, hf);
-        att_sm_end<false>(o0, l0, r);
+    if (lastb == 0 && ragged) zero_rows(0);
+    auto none = [](int) {};
+    auto kread = [&](int k, int off) {
+        if (k < 8) kf[k] = att_read_k(A, k, off);
+    };
+    auto vread = [&](int k, int half) {
+        if (k >= 8) vf[(k - 8) / 4][k & 3] = att_read_v<VT>(A, 2 * half + (k - 8) / 4, k & 3);
+    };
+#pragma unroll
+    for (int k = 0; k < 8; ++k) kread(k, 0);
+    att_region<false, true, false, false, -1>(t0, t1, qf[0], kf, vf, c, ones, none);
+    att_region<false, true, false, false, -1>(t1, t0, qf[1], kf, vf, c, ones, none);
+    if (lastb == 0 && ragged) {
+        att_mask(t0.s, kl, p.T, hf);
+        att_mask(t1.s, kl, p.T, hf);
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        kread(k, 32 * 256);
+        vread(k, 0);
     }
     if (FAST) {
-        if (lastb == 0 && ragged) att_mask(s1, key0, p.T, hf);
-        m1 = att_rowmax(s1) * c;
+        t0.m = att_rowmax(t0.s) * c;
+        t1.m = att_rowmax(t1.s) * c;
+#pragma unroll
+        for (int k = 0; k <= 17; ++k) att_exp(t0, k, c, ones);
+    } else {
+        att_softmax_safe(t0, c, ones);
     }
-    // Block n: sub-blocks u = 2n (fragments in the "a" registers) and 2n + 1 ("b").
+
+    constexpr int LDSK = VT ? 8 : 15;  // V reads after the K reads: 8 (V^T) or 16
     for (int n = 0; n < lastb; ++n) {
-        // ---- Y(2n): P V with vfa, next scores with kfb
-        {
-            att_pv(o0, vfa, pf0);
-            att_scores(s0, kfb, qf[0]);
-            const float r = att_sm<FAST>(s1, m1, l1, pf1, c);
-            att_sm_end<FAST>(o1, l1, r);
-        }
-        // Block n + 1 (K of sub-block 2n + 2, read in X(2n + 1)) landed for
-        // every wave; the slot of block n - 1 is free: issue block n + 3 there.
+        const uint32_t flip = att_flip(n);
+        // Y(2n)
+        att_region<FAST, true, true, true, LDSK>(t0, t1, qf[0], kf, vf, c, ones, none);
+        // Block n + 1 landed for every wave; the slot of block n - 1 is free.
         att_wait_vmcnt<8>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        att_issue(ld, wave, slot(n + 3), kb0 + (n + 3 < nkb ? n + 3 : lastb));
-        // ---- X(2n + 1): scores with kfb, P V with vfa; reads vfb, kfa
-        {
-            att_scores(s1, kfb, qf[1]);
-            att_pv(o1, vfa, pf1);
-            const float r = att_sm<FAST>(s0, m0, l0, pf0, c);
-            att_read_v(vfb, slot(n) + ATT_TILE, 1, lq, hf);
-            att_read_k(kfa, slot(n + 1), 0, lq, hf);
-            att_sm_end<FAST>(o0, l0, r);
+        att_issue_begin<VT>(p, ld, wave, lane);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) A.k[j] ^= flip;
+        // X(2n + 1)
+        att_region<FAST, true, true, true, -1>(t1, t0, qf[1], kf, vf, c, ones, [&](int k) {
+            kread(k, 0);
+            vread(k, 1);
+        });
+        // Y(2n + 1)
+        att_region<FAST, true, true, true, LDSK>(t0, t1, qf[0], kf, vf, c, ones, [&](int k) {
+            if (k & 1) att_issue_part<VT>(ld, k / 2);
+        });
+        att_issue_end(ld, att_flip(n + 3));
+        if (n + 1 == lastb && ragged) {
+            att_mask(t0.s, kl, p.T, hf);
+            zero_rows((lastb & 3) ^ ((lastb & 3) >> 1));
         }
-        // ---- Y(2n + 1): P V with vfb, next scores with kfa
-        {
-            att_pv(o0, vfb, pf0);
-            att_scores(s0, kfa, qf[0]);
-            const float r = att_sm<FAST>(s1, m1, l1, pf1, c);
-            att_sm_end<FAST>(o1, l1, r);
-        }
-        if (n + 1 == lastb && ragged) att_mask(s0, key0 + (n + 1) * ATT_KB, p.T, hf);
-        // ---- X(2n + 2): scores with kfa, P V with vfb; reads vfa, kfb
-        {
-            att_scores(s1, kfa, qf[1]);
-            att_pv(o1, vfb, pf1);
-            const float r = att_sm<FAST>(s0, m0, l0, pf0, c);
-            att_read_v(vfa, slot(n + 1) + ATT_TILE, 0, lq, hf);
-            att_read_k(kfb, slot(n + 1), 1, lq, hf);
-            att_sm_end<FAST>(o0, l0, r);
-        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) A.v[t] ^= flip;
+        // X(2n + 2)
+        att_region<FAST, true, true, true, -1>(t1, t0, qf[1], kf, vf, c, ones, [&](int k) {
+            kread(k, 32 * 256);
+            vread(k, 0);
+        });
     }
-    // Last block L: Y(2L), X(2L + 1), Y(2L + 1) and PV_1(2L + 1); its data
-    // landed at the last barrier (or the first), no further loads.
-    if (ragged) att_mask(s1, key0 + lastb * ATT_KB, p.T, hf);
-    {
-        att_pv(o0, vfa, pf0);
-        att_scores(s0, kfb, qf[0]);
-        const float r = att_sm<FAST>(s1, m1, l1, pf1, c);
-        att_sm_end<FAST>(o1, l1, r);
-    }
-    if (ragged) att_mask(s0, key0 + lastb * ATT_KB + 32, p.T, hf);
-    {
-        att_scores(s1, kfb, qf[1]);
-        att_pv(o1, vfa, pf1);
-        const float r = att_sm<FAST>(s0, m0, l0, pf0, c);
-        att_read_v(vfb, slot(lastb) + ATT_TILE, 1, lq, hf);
-        att_sm_end<FAST>(o0, l0, r);
-    }
-    if (ragged) att_mask(s1, key0 + lastb * ATT_KB + 32, p.T, hf);
-    {
-        att_pv(o0, vfb, pf0);
-        const float r = att_sm<FAST>(s1, m1, l1, pf1, c);
-        att_sm_end<FAST>(o1, l1, r);
-    }
-    att_pv(o1, vfb, pf1);
-    att_wait_vmcnt<0>();  // the clamped tail loads land before the LDS is reused or released
+    // Last block L: Y(2L), X(2L + 1), Y(2L + 1) without new scores, PV_1(2L + 1).
+    if (ragged) att_mask(t1.s, kl, p.T, hf);
+    att_region<FAST, true, true, true, LDSK>(t0, t1, qf[0], kf, vf, c, ones, none);
+    if (ragged) att_mask(t0.s, kl + 32, p.T, hf);
+    att_region<FAST, true, true, true, -1>(t1, t0, qf[1], kf, vf, c, ones, [&](int k) { vread(k, 1); });
+    if (ragged) att_mask(t1.s, kl + 32, p.T, hf);
+    att_region<FAST, false, true, true, 0>(t0, t1, qf[0], kf, vf, c, ones, none);
+    att_region<FAST, false, true, false, -1>(t1, t0, qf[1], kf, vf, c, ones, none);
+    att_wait_vmcnt<0>();  // the repeated tail loads land before the LDS is reused or released
 }
 
 // Bound on a lane's partial sum l after a FAST pass: below it, every P and
 // every |O| (for |V| < 2^63) stayed finite.
 constexpr float ATT_FAST_LMAX = 18446744073709551616.0f;  // 2^64
 
-template <bool QOUT>
+template <bool QOUT, bool VT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_attn_fwd(AttnArgs p) {
+    // The kernel's only LDS, so it starts at address 0 (AttAddr, AttLoader::lds).
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    __shared__ int redo[4];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lq = lane & 31, hf = lane >> 5;
@@ -476,52 +583,55 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int qblk = item % p.nq, h = (item / p.nq) % p.H, b = item / (p.nq * p.H);
     const int q0 = qblk * ATT_BQ + wave * 64;
 
+    // The first key blocks are in flight while Q is loaded.
+    const AttLoader ld = att_start<VT>(p, b, h, kb0, nkb, wave, lane);
     // Q^T operands: lane (q, hf) holds d [16j + 8hf, +8) of query q0 + 32t + q.
-    uint4 qf[2][8];
+    bf16x8_t qf[2][8];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         int qi = q0 + 32 * t + lq;
         qi = qi < p.S ? qi : p.S - 1;  // rows past the end: computed, not stored
         const uint16_t *qrow = p.q + ((int64_t)b * p.S + qi) * p.ldq + (int64_t)h * ATT_D + hf * 8;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) qf[t][j] = *reinterpret_cast<const uint4 *>(qrow + 16 * j);
+        for (int j = 0; j < 8; ++j) qf[t][j] = *reinterpret_cast<const bf16x8_t *>(qrow + 16 * j);
     }
     // Q^T is only ever an MFMA operand: keep it in accumulation registers, which
     // leaves the architectural ones to O, the scores, P and the softmax.
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            u32x4_t v = {qf[t][j].x, qf[t][j].y, qf[t][j].z, qf[t][j].w};
-            asm volatile("" : "+a"(v));
-            qf[t][j] = make_uint4(v.x, v.y, v.z, v.w);
-        }
+        for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(qf[t][j]));
 
-    const AttLoader ld = att_loader(p, b, h, wave, lane);
-    f32x16a_t o0[4], o1[4];
-    float m0, m1, l0, l1;
-    att_pass<true>(p, ld, lds, qf, wave, lq, hf, kb0, nkb, o0, o1, m0, m1, l0, l1);
+    AttTile t0, t1;
+    att_pass<true, VT>(p, ld, lds, qf, wave, lane, kb0, nkb, t0, t1);
+    float l0 = t0.l[0], l1 = t1.l[0];
     // Rerun the whole workgroup in the safe form when any wave's sums left
     // the range the fixed reference max guarantees (scores that grew by more
     // than ~64 in log2 units past their first sub-block's max).
-    if (threadIdx.x % 64 == 0) redo[wave] = 0;
     const bool bad = !(l0 < ATT_FAST_LMAX && l1 < ATT_FAST_LMAX);
-    if (__builtin_amdgcn_ballot_w64(bad) && lane == 0) redo[wave] = 1;
+    const int wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    __syncthreads();  // every wave is done with the rings
+    int *const redo = reinterpret_cast<int *>(lds);
+    if (lane == 0) redo[wave] = wave_bad;
     __syncthreads();
-    if (redo[0] | redo[1] | redo[2] | redo[3])
-        att_pass<false>(p, ld, lds, qf, wave, lq, hf, kb0, nkb, o0, o1, m0, m1, l0, l1);
+    if (__builtin_amdgcn_readfirstlane(redo[0] | redo[1] | redo[2] | redo[3])) {
+        __syncthreads();  // read by every wave before the rings are filled again
+        att_pass<false, VT>(p, att_start<VT>(p, b, h, kb0, nkb, wave, lane), lds, qf, wave, lane, kb0, nkb, t0, t1);
+        l0 = t0.l[0];
+        l1 = t1.l[0];
+    }
 
     // O = O^T / l: lane (q, hf) holds dims 32dt + 8(i/4) + 4hf + i%4 of its query.
     // A tail chunk writes the same bf16 rows into its part_o slot (256 x 128)
     // and (m, l) of each query into part_ml, for k_attn_merge.
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const f32x16a_t(&o)[4] = t ? o1 : o0;
+        const f32x16a_t(&o)[4] = t ? t1.o : t0.o;
         const float lf = t ? l1 : l0;
         const float lt = lf + __shfl_xor(lf, 32, 64);
         const float inv = 1.0f / lt;
         const int qi = q0 + 32 * t + lq;
-        if (qi >= p.S) continue;
+        const bool live = qi < p.S;  // the same for both half-waves of a query
         if (QOUT && tail < 0) {
             // MXFP8: the bf16 values the plain output would hold, quantized as
             // qim_mx_quantize does.  A 32-column block (dt) is this lane's 16
@@ -541,33 +651,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 const int e = mx_exponent(__uint_as_float(m));
                 const float s = mx_scale_operand(e);
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int64_t k = (int64_t)h * ATT_D + 32 * dt + 8 * g + 4 * hf;
-                    *reinterpret_cast<uint32_t *>(p.qcodes + att_code_offset(p, row, k)) =
-                        cvt_e4m3x4_scaled(f[4 * g], f[4 * g + 1], f[4 * g + 2], f[4 * g + 3], s);
+                for (int g = 0; g < 4; g += 2) {
+                    // Columns 8g + 4hf and 8(g + 1) + 4hf; after the exchange
+                    // the 8 of group g + hf.
+                    const auto c = __builtin_amdgcn_permlane32_swap(
+                        cvt_e4m3x4_scaled(f[4 * g], f[4 * g + 1], f[4 * g + 2], f[4 * g + 3], s),
+                        cvt_e4m3x4_scaled(f[4 * g + 4], f[4 * g + 5], f[4 * g + 6], f[4 * g + 7], s), false, false);
+                    const int64_t k = (int64_t)h * ATT_D + 32 * dt + 8 * (g + hf);
+                    if (live) *reinterpret_cast<uint2 *>(p.qcodes + att_code_offset(p, row, k)) = make_uint2(c[0], c[1]);
                 }
                 sc |= (uint32_t)e << (8 * dt);
             }
-            if (hf == 0)
+            if (live && hf == 0)
                 *reinterpret_cast<uint32_t *>(p.qscales + mx_scale_offset(row, 4 * h, (int64_t)p.H * ATT_D)) = sc;
             continue;
         }
         uint16_t *orow = p.o + ((int64_t)b * p.S + qi) * p.ldo + (int64_t)h * ATT_D;
+        bool vec16 = p.o_vec16;
         if (tail >= 0) {
             const int ql = wave * 64 + 32 * t + lq;
             orow = p.part_o + ((int64_t)tail * ATT_BQ + ql) * ATT_D;
-            if (hf == 0)
+            vec16 = true;
+            if (live && hf == 0)
                 *reinterpret_cast<float2 *>(p.part_ml + ((int64_t)tail * ATT_BQ + ql) * 2) =
-                    make_float2(t ? m1 : m0, lt);
+                    make_float2(t ? t1.m : t0.m, lt);
         }
+        // The half-waves exchange 4-column groups (8g + 4hf of an even and an odd
+        // g) so that each lane stores the 16 bytes of group g + hf: half as many
+        // stores, each instruction covering whole 32-byte sectors.
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d = 32 * dt + 8 * g + 4 * hf;
-                const uint2 w = make_uint2(pack_bf16x2(o[dt][4 * g + 0] * inv, o[dt][4 * g + 1] * inv),
-                                           pack_bf16x2(o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv));
-                *reinterpret_cast<uint2 *>(orow + d) = w;
+            for (int g = 0; g < 4; g += 2) {
+                const auto x = __builtin_amdgcn_permlane32_swap(pack_bf16x2(o[dt][4 * g + 0] * inv, o[dt][4 * g + 1] * inv),
+                                                                pack_bf16x2(o[dt][4 * g + 4] * inv, o[dt][4 * g + 5] * inv),
+                                                                false, false);
+                const auto y = __builtin_amdgcn_permlane32_swap(pack_bf16x2(o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv),
+                                                                pack_bf16x2(o[dt][4 * g + 6] * inv, o[dt][4 * g + 7] * inv),
+                                                                false, false);
+                uint16_t *at = orow + 32 * dt + 8 * (g + hf);
+                if (live && vec16) {
+                    *reinterpret_cast<uint4 *>(at) = make_uint4(x[0], y[0], x[1], y[1]);
+                } else if (live) {  // ldo need only be a multiple of 4 elements
+                    *reinterpret_cast<uint2 *>(at) = make_uint2(x[0], y[0]);
+                    *reinterpret_cast<uint2 *>(at + 4) = make_uint2(x[1], y[1]);
+                }
             }
     }
 }
@@ -655,6 +783,12 @@ using namespace qim;
 namespace qim {
 
 constexpr int ATT_MIN_CHUNK = 8;
+// Most queries per image for which V is read as rows: the transposing reads
+// take two instructions per fragment, the transpose pass one trip of V through
+// memory, and the reads are repeated by every query block.  Rows against V^T:
+// S 1024, T 1101, B 2, H 32 49.9 / 59.6 us; S 4352 264 / 266 us; S 8192 797 / 790
+// us; S 16640 2889 / 2848 us.
+constexpr int64_t ATT_VROWS_MAX_S = 8192;
 
 AttPlan att_plan(int64_t B, int64_t S, int64_t T, int64_t H) {
     const int64_t nq = (S + ATT_BQ - 1) / ATT_BQ, nkb = (T + ATT_KB - 1) / ATT_KB, W = B * H * nq;
@@ -715,19 +849,25 @@ int attention_run(const char *who, const void *q, int64_t ldq, const void *k, in
     QIM_REQUIRE(workspace_bytes >= pl.total(), QIM_ERR_ARG,
                 "%s: workspace of %lld bytes, this problem needs %lld (qim_attention_workspace_bytes)", who,
                 (long long)workspace_bytes, (long long)pl.total());
-    static std::atomic<bool> configured[2][QIM_MAX_DEVICES] = {};
-    const void *fwd = qcodes ? reinterpret_cast<const void *>(&k_attn_fwd<true>)
-                             : reinterpret_cast<const void *>(&k_attn_fwd<false>);
-    if (const int rc = reserve_lds(fwd, ATT_LDS, configured[qcodes ? 1 : 0], who)) return rc;
+    // V rows read through the transposing LDS reads, or V^T tiles: from the
+    // workspace when v is null, else made here.
+    const bool vt = !v || S > ATT_VROWS_MAX_S || ldv >= (1ll << 25);  // (32-bit row offsets)
+    static std::atomic<bool> configured[4][QIM_MAX_DEVICES] = {};
+    void (*const fwd)(AttnArgs) = qcodes ? (vt ? k_attn_fwd<true, true> : k_attn_fwd<true, false>)
+                                         : (vt ? k_attn_fwd<false, true> : k_attn_fwd<false, false>);
+    if (const int rc = reserve_lds(reinterpret_cast<const void *>(fwd), ATT_LDS, configured[(qcodes ? 2 : 0) + vt], who))
+        return rc;
     hipStream_t st = as_stream(stream);
     uint8_t *ws = static_cast<uint8_t *>(workspace);
-    if (v)
+    if (v && vt)
         launch(k_attn_vt, dim3((unsigned)nkb, (unsigned)H, (unsigned)B), dim3(256), 0, st,
                            (const uint16_t *)v, ldv, (uint16_t *)ws, (int)T, (int)H, (int)nkb);
     AttnArgs a{};
     a.q = (const uint16_t *)q;
     a.k = (const uint16_t *)k;
     a.vt = (const uint16_t *)ws;
+    a.v = (const uint16_t *)v;
+    a.ldv = ldv;
     a.o = (uint16_t *)o;
     a.ldq = ldq;
     a.ldk = ldk;
@@ -749,11 +889,9 @@ int attention_run(const char *who, const void *q, int64_t ldq, const void *k, in
     a.qscales = static_cast<uint8_t *>(qscales);
     a.Mp = (M + 127) / 128 * 128;
     a.tiled = tiled;
+    a.o_vec16 = o && aligned16(o) && ldo % 8 == 0;
     const int64_t nwg = pl.nfull + pl.ntail * pl.nsplit;
-    if (qcodes)
-        launch(k_attn_fwd<true>, dim3((unsigned)nwg), dim3(256), ATT_LDS, st, a);
-    else
-        launch(k_attn_fwd<false>, dim3((unsigned)nwg), dim3(256), ATT_LDS, st, a);
+    launch(fwd, dim3((unsigned)nwg), dim3(256), ATT_LDS, st, a);
     if (pl.ntail) {
         const int64_t threads = pl.ntail * ATT_BQ * (ATT_D / 8);
         launch(k_attn_merge, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, a);

@@ -139,3 +139,40 @@ def test_attention_rejects_other_head_dims(dev):
     x = torch.zeros(1, 8, 1, 64, dtype=torch.bfloat16, device=dev)
     with pytest.raises(_native.Unsupported):
         attention.attention(x, x, x)
+
+
+@pytest.mark.parametrize("t", [1, 31, 33, 64, 65, 100, 161, 225, 290, 333, 511])
+def test_attention_v_rows_against_v_tiles(dev, t):
+    """V read as rows (up to 8192 queries) and as transposed tiles (more): the
+    same products in the same order, so the same bits for the same queries, at
+    partial sub-blocks and blocks, with an infinity and a NaN in V's last row
+    (which the rows past it must not touch), in the plain and the MXFP8 form."""
+    say("attention v rows / tiles", t)
+    g = torch.Generator().manual_seed(t)
+    q, k, v = (bf16_randn(g, (1, n, 2, 128)).to(dev) for n in (8448, t, t))
+    v[0, -1, 0, 5], v[0, -1, 1, 7] = float("inf"), float("nan")
+    tiles = attention.attention(q, k, v)
+    rows = attention.attention(q[0, :1024].unsqueeze(0), k, v)
+    assert torch.equal(tiles[:, :1024].contiguous().view(torch.int16), rows.view(torch.int16))
+    assert not torch.isfinite(rows[0, :, 0, 5].float()).any() and torch.isnan(rows[0, :, 1, 7].float()).all()
+    assert torch.isfinite(rows[0, :, 0, 6:].float()).all() and torch.isfinite(rows[0, :, 1, 8:].float()).all()
+    v[0, -1, 0, 5], v[0, -1, 1, 7] = 1.0, -1.0
+    tq, rq = attention.attention_mxfp8(q, k, v, tiled=False), attention.attention_mxfp8(q[0, :1024].unsqueeze(0), k, v,
+                                                                                      tiled=False)
+    assert torch.equal(tq.values[:1024].view(torch.uint8), rq.values.view(torch.uint8))
+    ref = mxfp8.quantize(attention.attention(q, k, v).view(8448, 256))
+    assert torch.equal(tq.values.view(torch.uint8), ref.values.view(torch.uint8))
+    assert torch.equal(tq.scales.view(torch.uint8), ref.scales.view(torch.uint8))
+
+
+def test_attention_output_stride_of_four(dev):
+    """An output whose rows are 8- but not 16-byte aligned, and one that is."""
+    say("attention output stride")
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (bf16_randn(g, (1, n, 3, 128)).to(dev) for n in (300, 200, 200))
+    want = attention.attention(q, k, v)
+    for pad in (4, 8):
+        wide = torch.zeros(1, 300, 384 + pad, device=dev, dtype=torch.bfloat16)
+        out = wide[:, :, :384].unflatten(-1, (3, 128))
+        attention.attention(q, k, v, out=out)
+        assert torch.equal(out, want) and not wide[:, :, 384:].any()

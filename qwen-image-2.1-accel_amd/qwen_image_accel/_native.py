@@ -81,6 +81,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_functions = {}  # entry point name -> ctypes function, filled by lib()
 _lock = threading.Lock()
 calls = {}  # entry point name -> number of successful launches (tests use it)
 
@@ -102,13 +103,14 @@ def lib():
                     fn = getattr(handle, name)
                     fn.restype = res
                     fn.argtypes = args
+                    _functions[name] = fn
                 _lib = handle
     return _lib
 
 
 def call(name, *args):
     """Call an entry point; raise Unsupported / QimError on a nonzero status."""
-    rc = getattr(lib(), name)(*args)
+    rc = (_functions.get(name) or getattr(lib(), name))(*args)
     if rc != QIM_OK:
         msg = lib().qim_last_error().decode(errors="replace")
         if rc in (QIM_ERR_SHAPE, QIM_ERR_LAYOUT):
@@ -119,12 +121,26 @@ def call(name, *args):
 
 def ptr(t):
     """Device address of a tensor (None stays NULL)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+def complex_ptr(t):
+    """Device address of a contiguous complex tensor's (re, im) pairs.  A lazily
+    conjugated tensor does not hold its values: torch.view_as_real refuses it."""
+    return torch.view_as_real(t).data_ptr() if t.is_conj() else t.data_ptr()
+
+
+# The raw handle of a device's current stream: 0.06 us, where building a
+# torch.cuda.Stream object to read it from takes 2 us (of a ~10 us call).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream(device=None):
     """The current torch stream of `device` as a hipStream_t."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = None if device is None else torch.device(device).index
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def loaded_hip_runtimes():

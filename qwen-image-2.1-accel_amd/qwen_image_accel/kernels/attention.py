@@ -49,10 +49,9 @@ def prepare_attention_inputs(q, k, v, norm_q, norm_k, freqs, cached_k, cached_v)
     oq = torch.empty((b, s, h, d), device=q.device, dtype=q.dtype)
     ok = torch.empty((b, s + p, h, d), device=q.device, dtype=q.dtype)
     ov = torch.empty_like(ok)
-    f = torch.view_as_real(freqs)
     _native.call("qim_qk_norm_rope_pack", _native.ptr(q), _native.ptr(k), _native.ptr(v),
                  _native.ptr(cached_k) if p else None, _native.ptr(cached_v) if p else None,
-                 _native.ptr(norm_q.weight), _native.ptr(norm_k.weight), _native.ptr(f),
+                 _native.ptr(norm_q.weight), _native.ptr(norm_k.weight), _native.complex_ptr(freqs),
                  _native.ptr(oq), _native.ptr(ok), _native.ptr(ov), b, s, p, h, d, ldt,
                  float(norm_q.eps), float(norm_k.eps), _native.stream(q.device))
     return oq, ok, ov
@@ -61,8 +60,12 @@ def prepare_attention_inputs(q, k, v, norm_q, norm_k, freqs, cached_k, cached_v)
 def workspace(b, s, t, h, device, d=128):
     """A workspace for ``attention`` / ``attention_mxfp8`` of this shape (V^T
     tiles first, then the split items' partial results)."""
-    with torch.cuda.device(device):
+    device = torch.device(device)
+    if device.index is None or device.index == torch.cuda.current_device():
         nbytes = _native.lib().qim_attention_workspace_bytes(b, s, t, h, d)
+    else:  # the split depends on the device's CU count
+        with torch.cuda.device(device):
+            nbytes = _native.lib().qim_attention_workspace_bytes(b, s, t, h, d)
     if nbytes <= 0:
         raise _native.Unsupported("attention", _native.QIM_ERR_SHAPE, f"head dim {d} (128 only)")
     return torch.empty(nbytes, device=device, dtype=torch.uint8)
@@ -144,9 +147,9 @@ def qk_norm_rope(q, k, weight_q, weight_k, freqs, eps_q=1e-6, eps_k=1e-6, heads=
             raise _native.Unsupported("qk_norm_rope", _native.QIM_ERR_LAYOUT, "q/k layout")
     oq = torch.empty((b, s, h, d), device=q.device, dtype=torch.bfloat16)
     ok = torch.empty_like(oq)
-    f = torch.view_as_real(freqs.contiguous())
+    f = freqs.contiguous()
     _native.call("qim_qk_norm_rope_pack", _native.ptr(q), _native.ptr(k), None, None, None,
-                 _native.ptr(weight_q), _native.ptr(weight_k), _native.ptr(f), _native.ptr(oq),
+                 _native.ptr(weight_q), _native.ptr(weight_k), _native.complex_ptr(f), _native.ptr(oq),
                  _native.ptr(ok), None, b, s, 0, h, d, ldt, float(eps_q), float(eps_k),
                  _native.stream(q.device))
     return oq, ok

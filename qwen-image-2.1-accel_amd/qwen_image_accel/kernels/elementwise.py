@@ -60,7 +60,7 @@ def rope_qk(q, k, freqs):
     b, s, h, d = q.shape
     if d not in HEAD_DIMS:
         raise _native.Unsupported("rope_qk", _native.QIM_ERR_SHAPE, f"head dim {d}")
-    f = torch.view_as_real(freqs.contiguous())
-    _native.call("qim_rope_qk", _native.ptr(q), _native.ptr(k), _native.ptr(f),
+    f = freqs.contiguous()
+    _native.call("qim_rope_qk", _native.ptr(q), _native.ptr(k), _native.complex_ptr(f),
                  _native.ptr(out_q), _native.ptr(out_k), b, s, h, d, _native.stream(q.device))
     return out_q, out_k

@@ -50,9 +50,9 @@ def mx_matmul_qk_norm_rope(activation, weight_fp8, weight_scale, weight_q, weigh
     if out.dtype != torch.bfloat16 or out.stride(-1) != 1 or out.shape != (m, n):
         raise ValueError("out must be a bf16 (rows, N) tensor with unit column stride")
     layouts = (_native.GEMM_A_TILED if a.tiled else 0) | (_native.GEMM_B_TILED if weight_tiled else 0)
-    f = torch.view_as_real(freqs.contiguous())
+    f = freqs.contiguous()
     args = (_native.ptr(a.values), _native.ptr(a.scales), _native.ptr(w), _native.ptr(weight_scale), m, k, heads,
-            layouts, _native.ptr(weight_q), _native.ptr(weight_k), _native.ptr(f), seq, float(eps_q), float(eps_k),
+            layouts, _native.ptr(weight_q), _native.ptr(weight_k), _native.complex_ptr(f), seq, float(eps_q), float(eps_k),
             _native.ptr(out), out.stride(0))
     if vt is None:
         _native.call("qim_mxfp8_gemm_qk_norm_rope", *args, _native.stream(out.device))

@@ -29,31 +29,27 @@ def _eager(x, scale, norm, shift, gate, residual, add_one):
     return y
 
 
-def _vec_ok(v, x):
-    b, _, d = x.shape
-    return (v is None or (v.shape == (b, 1, d) and v.dtype == torch.bfloat16
-                          and v.device == x.device and v.is_contiguous()))
+def _vec_ok(v, shape, device):
+    return (v is None or (v.shape == shape and v.dtype == torch.bfloat16
+                          and v.device == device and v.is_contiguous()))
 
 
 def native_supported(x, scale, norm, shift=None, gate=None, residual=None):
     """True when the HIP kernel handles these operands (the guard of
     kernels/layernorm.py:59-72, generalised in D)."""
-    if (x.ndim != 3 or not x.is_cuda or x.dtype != torch.bfloat16 or not x.is_contiguous()
-            or x.numel() == 0):
+    if x.ndim != 3 or not x.is_cuda or x.dtype != torch.bfloat16 or not x.is_contiguous():
         return False
-    d = x.shape[-1]
-    if d % 8 or d > 16384:
+    b, s, d = x.shape
+    if b * s * d == 0 or d % 8 or d > 16384:
         return False
-    if not (_vec_ok(scale, x) and _vec_ok(shift, x) and _vec_ok(gate, x)):
-        return False
-    if scale is None:
+    shape, device = (b, 1, d), x.device
+    if scale is None or not (_vec_ok(scale, shape, device) and _vec_ok(shift, shape, device)
+                             and _vec_ok(gate, shape, device)):
         return False
     if residual is not None and (residual.shape != x.shape or residual.dtype != torch.bfloat16
-                                 or residual.device != x.device or not residual.is_contiguous()):
+                                 or residual.device != device or not residual.is_contiguous()):
         return False
-    if getattr(norm, "elementwise_affine", False) or tuple(norm.normalized_shape) != (d,):
-        return False
-    return True
+    return not getattr(norm, "elementwise_affine", False) and tuple(norm.normalized_shape) == (d,)
 
 
 def _flags(add_one):

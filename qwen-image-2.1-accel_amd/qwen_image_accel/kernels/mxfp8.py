@@ -51,10 +51,9 @@ def empty_quantized(rows, k, device, shape=None, tiled=False):
     """Allocate the output buffers of a quantization of (rows, k)."""
     padded = padded_rows(rows)
     q = torch.empty((padded, k), device=device, dtype=torch.float8_e4m3fn)
-    s = torch.empty(padded * k // BLOCK, device=device, dtype=torch.uint8)
+    s = torch.empty(padded * k // BLOCK, device=device, dtype=torch.float8_e8m0fnu)
     kind = TiledQuantized if tiled else Quantized
-    return kind(q, s.view(torch.float8_e8m0fnu), rows,
-                torch.Size((rows, k)) if shape is None else torch.Size(shape))
+    return kind(q, s, rows, torch.Size((rows, k)) if shape is None else torch.Size(shape))
 
 
 def quantize(x, *, tiled=False):

@@ -78,6 +78,7 @@ struct GemmArgs {
     float *ws;
     int ksplit;
     int qrows, qcols;  // a grid of quarter tiles only: its rows and columns (qrows 0 otherwise)
+    int tile_rows;     // rows of a whole tile: 256, or 192 (k_mx_gemm_192; tiles_m counts those)
 };
 
 // qim_mxfp8_gemm_qk_norm_rope_vt: the QK-norm + RoPE epilogue whose V columns
@@ -1136,6 +1137,187 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     quarter_tile<EPI, NP>(p, smem, xcd * base + (xcd < rem ? xcd : rem) + (int)(blockIdx.x >> 3));
 }
 
+// ---------------------------------------------------------- 192-row tiles --
+// Whole tiles of 192 x 256 for grids of 256 x 256 tiles that leave CUs idle in
+// their one round while three quarters of a tile per CU would not (gemm_plan):
+// 2381 x 4096 x 12288 has 160 whole tiles or 208 of these, 109.3 -> 102.1 us (2.35
+// PFLOP/s: from there the power limit holds it, as it does the largest grids).  4 waves side by side, each
+// a 192 x 64 block of 6 x 2 MFMA tiles (the epilogues work in 64-row halves of a
+// wave, so the rows stay together).  A stage's 92 KiB of LDS traffic (28 KiB of
+// DMA writes, 64 KiB of fragment reads) against 768 MFMA cycles is the most the
+// LDS moves in that time.  The ring, its waits and the schedule are the whole
+// tile's; a 192-row tile may start in the middle of a 128-row scale chunk or a
+// 256-row super-block of the tiled layout, so each A load has its own K step and
+// the six scale dwords come in three 8-byte reads.  (A fifth ring slot: the same
+// times within 1 %.)
+constexpr int TBM = 192, TA_BYTES = TBM * BK;
+constexpr int TSTAGE_BYTES = TA_BYTES + TILE_BYTES + 2 * SCALE_BYTES;  // 30 KiB
+constexpr int TLDS_BYTES = NSTAGE * TSTAGE_BYTES;                      // 120 KiB
+constexpr int TLOADS_EVEN = 9, TLOADS_ODD = 7;  // per wave per stage: 3 A + 4 B (16 B), 2 of scales (4 B)
+
+struct TPlan {
+    uint32_t a[3], b[4], astep[3], bstep;
+    uint32_t sc[2];
+    const uint8_t *sc_base[2];
+    uint32_t sa[3], sb;  // LDS offsets, in a stage, of this lane's scale dword pairs
+    int wave;
+};
+
+__device__ __forceinline__ TPlan make_tplan(const GemmArgs &p, int64_t m0, int64_t n0) {
+    TPlan L;
+    const int lane = threadIdx.x & 63, lr = lane & 31;
+    L.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int grp = (L.wave * 3 + j) * 16;
+        const int64_t rg = m0 + grp <= p.Mp - 16 ? m0 + grp : p.Mp - 16;
+        L.a[j] = opnd_offset(m0, grp, lane, p.Mp, p.K, p.a_tiled);
+        L.astep[j] = opnd_step(rg, p.Mp, p.a_tiled);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) L.b[j] = opnd_offset(n0, (L.wave * 4 + j) * 16, lane, p.N, p.K, p.b_tiled);
+    L.bstep = opnd_step(n0, p.N, p.b_tiled);
+    const int64_t kt = p.K / 128;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int idx = L.wave * 2 + j;  // 0..3: A scale quarter, 4..7: B scale quarter
+        const int off = (idx & 3) * 256 + lane * 4;
+        int64_t grow = (idx < 4 ? m0 : n0) / 128 + (off >> 9);
+        if (idx < 4 && grow >= p.Mp / 128) grow = p.Mp / 128 - 1;  // rows past Mp: never stored
+        L.sc_base[j] = idx < 4 ? p.as : p.bs;
+        L.sc[j] = (uint32_t)(grow * kt * 512 + (off & 511));
+    }
+    // Row tiles 2u, 2u + 1 are the 32-row groups pt, pt + 1 from the start of
+    // m0's scale chunk; pt is even, so both dwords are in one aligned 8 bytes.
+    const int first = (int)(m0 & 127) / 32;  // 0 or 2
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        const int pt = first + 2 * u;
+        L.sa[u] = (uint32_t)(TA_BYTES + TILE_BYTES + (pt >> 2) * 512 + lr * 16 + (pt & 3) * 4);
+    }
+    L.sb = (uint32_t)(TA_BYTES + TILE_BYTES + SCALE_BYTES + (L.wave >> 1) * 512 + lr * 16 + (L.wave & 1) * 8);
+    return L;
+}
+
+template <bool SCALES>
+__device__ __forceinline__ void issue_tstage(const GemmArgs &p, const TPlan &L, uint8_t *slot, int s) {
+    const uint32_t kb = (uint32_t)s * L.bstep, base = lds_addr(slot);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) dma16(p.aq, L.a[j] + (uint32_t)s * L.astep[j], base + (L.wave * 3 + j) * 1024);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dma16(p.bq, L.b[j] + kb, base + TA_BYTES + (L.wave * 4 + j) * 1024);
+    if constexpr (SCALES) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            dma4(L.sc_base[j], L.sc[j] + (uint32_t)(s >> 1) * 512,
+                 base + TA_BYTES + TILE_BYTES + (L.wave * 2 + j) * 256);
+    }
+}
+
+struct TFrags {
+    i32x8_t a[6], b[2];
+    uint2 sa[3], sb;
+};
+
+__device__ __forceinline__ void read_tscales(const uint8_t *slot, const TPlan &L, TFrags &f) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) f.sa[u] = *reinterpret_cast<const uint2 *>(slot + L.sa[u]);
+    f.sb = *reinterpret_cast<const uint2 *>(slot + L.sb);
+}
+
+// One stage: as pipeline_step, 12 MFMAs with 7 or 9 DMA issues of stage s + 4 and
+// the reads of stage s + 1 between them.  The wait before the barrier covers
+// this wave's reads of the slot that stage s + 4 overwrites.
+template <int PAR>
+__device__ __forceinline__ void tstep(const GemmArgs &p, const TPlan &L, uint8_t *lds, int s, int S,
+                                      f32x16_t (&acc)[6][2], const TFrags &cur, TFrags &nxt, int lr, int kh) {
+    int sa[6], sb[2];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        sa[2 * u] = (int)(cur.sa[u].x >> (8 * kh));
+        sa[2 * u + 1] = (int)(cur.sa[u].y >> (8 * kh));
+    }
+    sb[0] = (int)(cur.sb.x >> (8 * kh));
+    sb[1] = (int)(cur.sb.y >> (8 * kh));
+    const uint8_t *next = lds + ((s + 1) & 3) * TSTAGE_BYTES;  // stale at the last stage; unused then
+    const uint8_t *nextb = next + TA_BYTES;
+    const int sl = s + 4 < S ? s + 4 : S - 1;  // stage to load (clamped)
+    const uint32_t kb = (uint32_t)sl * L.bstep, gofs = (uint32_t)(sl >> 1) * 512;
+    const uint32_t fb = lds_addr(lds + (s & 3) * TSTAGE_BYTES), fbb = fb + TA_BYTES, fbs = fbb + TILE_BYTES;
+    const uint32_t w3 = L.wave * 3, w4 = L.wave * 4;
+    const int rb = L.wave * 64 + lr;
+#define QIM_TMF(i, j)                                                                                         \
+    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(cur.a[i], cur.b[j], acc[i][j], 0, 0, PAR * 2, \
+                                                                sa[i], PAR * 2, sb[j])
+#define QIM_TSTEP(mi, mj, work) QIM_TMF(mi, mj); QIM_SCHED(); work; QIM_SCHED()
+    QIM_TMF(0, 0);
+    QIM_SCHED();
+    wait_vmcnt<TLOADS_EVEN + TLOADS_ODD>();  // stage s + 1 landed
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    QIM_SCHED();
+    QIM_TSTEP(0, 1, dma16(p.aq, L.a[0] + (uint32_t)sl * L.astep[0], fb + (w3 + 0) * 1024);
+              nxt.a[0] = read_tile(next, lr, kh));
+    QIM_TSTEP(1, 0, dma16(p.aq, L.a[1] + (uint32_t)sl * L.astep[1], fb + (w3 + 1) * 1024);
+              nxt.b[0] = read_tile(nextb, rb, kh));
+    QIM_TSTEP(1, 1, dma16(p.aq, L.a[2] + (uint32_t)sl * L.astep[2], fb + (w3 + 2) * 1024);
+              nxt.b[1] = read_tile(nextb, rb + 32, kh));
+    QIM_TSTEP(2, 0, dma16(p.bq, L.b[0] + kb, fbb + (w4 + 0) * 1024);
+              if constexpr (PAR == 0) {
+                  nxt.sa[0] = cur.sa[0]; nxt.sa[1] = cur.sa[1]; nxt.sa[2] = cur.sa[2]; nxt.sb = cur.sb;
+              } else read_tscales(next, L, nxt));
+    QIM_TSTEP(2, 1, dma16(p.bq, L.b[1] + kb, fbb + (w4 + 1) * 1024); nxt.a[1] = read_tile(next, 32 + lr, kh));
+    QIM_TSTEP(3, 0, dma16(p.bq, L.b[2] + kb, fbb + (w4 + 2) * 1024); nxt.a[2] = read_tile(next, 64 + lr, kh));
+    QIM_TSTEP(3, 1, dma16(p.bq, L.b[3] + kb, fbb + (w4 + 3) * 1024); nxt.a[3] = read_tile(next, 96 + lr, kh));
+    QIM_TSTEP(4, 0, if constexpr (PAR == 0) dma4(L.sc_base[0], L.sc[0] + gofs, fbs + (L.wave * 2 + 0) * 256);
+              nxt.a[4] = read_tile(next, 128 + lr, kh));
+    QIM_TSTEP(4, 1, if constexpr (PAR == 0) dma4(L.sc_base[1], L.sc[1] + gofs, fbs + (L.wave * 2 + 1) * 256);
+              nxt.a[5] = read_tile(next, 160 + lr, kh));
+    QIM_TMF(5, 0);
+    QIM_TMF(5, 1);
+    QIM_SCHED();
+#undef QIM_TSTEP
+#undef QIM_TMF
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_mx_gemm_192(GemmArgs p) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    // Contiguous ranges of tiles per XCD, as in k_mx_gemm_quarter.
+    const int n = gridDim.x, xcd = blockIdx.x & 7, base = n >> 3, rem = n & 7;
+    int tm, tn;
+    tile_coords(p, xcd * base + (xcd < rem ? xcd : rem) + (int)(blockIdx.x >> 3), tm, tn);
+    const int64_t m0 = (int64_t)tm * TBM, n0 = (int64_t)tn * BN;
+    const int lane = threadIdx.x & 63, lr = lane & 31, kh = lane >> 5;
+    const int S = (int)(p.K / BK);
+    f32x16_t acc[6][2];
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x16_t{};
+    const TPlan L = make_tplan(p, m0, n0);
+    uint8_t *const lds = smem;
+    issue_tstage<true>(p, L, lds, 0);
+    issue_tstage<false>(p, L, lds + TSTAGE_BYTES, 1);  // S is even
+    issue_tstage<true>(p, L, lds + 2 * TSTAGE_BYTES, 2 < S ? 2 : S - 1);
+    issue_tstage<false>(p, L, lds + 3 * TSTAGE_BYTES, 3 < S ? 3 : S - 1);
+    wait_vmcnt<TLOADS_ODD + TLOADS_EVEN + TLOADS_ODD>();  // stage 0 landed
+    block_barrier();
+    TFrags fa, fb;
+#pragma unroll
+    for (int t = 0; t < 6; ++t) fa.a[t] = read_tile(lds, t * 32 + lr, kh);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) fa.b[t] = read_tile(lds + TA_BYTES, L.wave * 64 + t * 32 + lr, kh);
+    read_tscales(lds, L, fa);
+    for (int s = 0; s < S; s += 2) {
+        tstep<0>(p, L, lds, s, S, acc, fa, fb, lr, kh);
+        tstep<1>(p, L, lds, s + 1, S, acc, fb, fa, lr, kh);
+    }
+    wait_vmcnt<0>();  // the clamped tail loads must land before LDS is reused
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    block_barrier();
+    epilogue<EPI, 6, 2>(p, acc, lds, nullptr, m0, n0 + L.wave * 64, lane, L.wave);
+}
+
 // The split-K second launch: sums each quarter tile's ksplit partials in order
 // kp = 0, 1, ... and runs the plain, bias or gated-residual epilogue.  One
 // lane per 8 columns of a row (16 lanes per row of a quarter, 16 rows per
@@ -1235,6 +1417,14 @@ static int launch_gemm(const GemmArgs &a, hipStream_t st) {
         const int64_t units = a.quarters * split;
         if (const int rc = units <= plan_cus() ? launch_quarters<EPI, 4>(a, units, st) : launch_quarters<EPI, 2>(a, units, st))
             return rc;
+    } else if (a.tile_rows == TBM) {
+        if constexpr (ring_offset<EPI>() == 0) {
+            static std::atomic<bool> configured192[QIM_MAX_DEVICES] = {};
+            if (const int rc = reserve_lds(reinterpret_cast<const void *>(&k_mx_gemm_192<EPI>), TLDS_BYTES, configured192,
+                                           "qim_mxfp8_gemm"))
+                return rc;
+            launch(k_mx_gemm_192<EPI>, dim3((unsigned)a.main_tiles), dim3(256), TLDS_BYTES, st, a);
+        }
     } else {
         constexpr int lds_bytes = LDS_BYTES + ring_offset<EPI>();
         if (const int rc = reserve_lds(reinterpret_cast<const void *>(&k_mx_gemm<EPI>), lds_bytes, configured,
@@ -1256,10 +1446,12 @@ static bool splits_k(int epilogue) {
 
 // How one problem runs: main_tiles whole tiles, then the quarter tiles of the
 // other whole tiles (times ksplit) and those of a last 128-column block; or,
-// with qrows set, quarters = qrows x qcols quarter tiles only (times ksplit).
+// with qrows set, quarters = qrows x qcols quarter tiles only (times ksplit); or,
+// with tile_rows 192, main_tiles tiles of 192 x 256 only.
 struct GemmPlan {
     int64_t main_tiles, quarters, qrows, qcols;
     int ksplit;
+    int tile_rows = BM;
     int64_t ws_bytes() const { return ksplit > 1 ? quarters * ksplit * (int64_t)QPART_WORDS * 4 : 0; }
 };
 
@@ -1295,6 +1487,18 @@ static GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int epilogue) {
         const int64_t q = qrows * qcols;
         return GemmPlan{0, q, qrows, qcols, splits_k(epilogue) ? quarter_ksplit(q, M, N, pairs) : 1};
     }
+    // One partial round of whole tiles: tiles of 192 x 256 instead, when those fit
+    // one round too (a 192-row tile runs at the whole tile's rate and takes
+    // three quarters of its work).  256- against 192-row tiles, operands rotated:
+    // 1280 x 9216 x 3072 (180 / 252 tiles) 35.5 -> 32.9 us, 2381 x 4096 x 12288 (160 /
+    // 208) 109.3 -> 102.1, 3072 x 4096 x 4096 (192 / 256) 44.2 -> 40.7, x 12288 117.7 ->
+    // 113.2, 2816 x 3072 x 3072 (132 / 180) 29.3 -> 26.4 us.  Above 256 of them a second
+    // round costs more than the whole tiles' one.  The SwiGLU epilogues keep whole
+    // tiles: their scale staging and SiLU table are laid out for 128 x 128 waves.
+    const int64_t tiles192 = (Mp + TBM - 1) / TBM * tiles_n;
+    if (tiles < cus && tiles192 <= cus && tiles_n * BN == N && epilogue != QIM_EPI_SWIGLU &&
+        epilogue != QIM_EPI_SWIGLU_QUANT)
+        return GemmPlan{tiles192, 0, 0, 0, 1, TBM};
     const int64_t main = main_tile_count(tiles);
     GemmPlan pl{main, 4 * (tiles - main), 0, 0, 1};
     // K-splits of the tail's quarter tiles: as many as fill the CUs' one round
@@ -1374,6 +1578,8 @@ static int gemm_run(const void *aq, const void *as, const void *bq, const void *
     a.quarters = (int)pl.quarters;
     a.qrows = (int)pl.qrows;
     a.qcols = (int)pl.qcols;
+    a.tile_rows = pl.tile_rows;
+    if (pl.tile_rows != BM) a.tiles_m = (int)((Mp + pl.tile_rows - 1) / pl.tile_rows);
     if (ws) {
         QIM_REQUIRE(aligned16(ws), QIM_ERR_LAYOUT, "qim_mxfp8_gemm_ws: ws must be 16-byte aligned");
         if (pl.ksplit > 1 && ws_bytes >= pl.ws_bytes()) {

@@ -258,7 +258,7 @@ __device__ __forceinline__ void read_frags(const uint8_t *slot, int wm, int wn, 
 // move anything across QIM_SCHED()).  With one wave per SIMD the MFMA pipe
 // idles whenever the wave stalls, so the 16 MFMAs of stage s (operands in
 // `cur`) are spread around everything else the stage has to do:
-//   MFMA 0 | wait for stage s+1's DMA, barrier | MFMA 1-3, each followed by a
+//   MFMA 0 | wait for stage s+1's DMA and this wave's reads of stage s, barrier | MFMA 1-3, each followed by a
 //   third of the 10 DMA issues of stage s+4 | MFMA 4-15, each followed by two
 //   of the 24 LDS reads of stage s+1's operands into `nxt`.
 // The scale dwords hold the exponents of K blocks 0..3 of the stage's 128-K
@@ -292,7 +292,7 @@ __device__ __forceinline__ void pipeline_step(const GemmArgs &p, const LoadPlan 
     QIM_MF(0, 0);
     QIM_SCHED();
     wait_vmcnt<LOADS_EVEN + LOADS_ODD>();
-    block_barrier();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     QIM_SCHED();
     QIM_STEP(0, 1, dma16(p.aq, L.a[0] + ka, fb + (w4 + 0) * 1024));
     // The next stage's scales: the same 128-K group after an even stage (kept

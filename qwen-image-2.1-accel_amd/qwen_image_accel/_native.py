@@ -126,8 +126,9 @@ def ptr(t):
 
 def complex_ptr(t):
     """Device address of a contiguous complex tensor's (re, im) pairs.  A lazily
-    conjugated tensor does not hold its values: torch.view_as_real refuses it."""
-    return torch.view_as_real(t).data_ptr() if t.is_conj() else t.data_ptr()
+    conjugated tensor does not hold its values, and a real one has no pairs:
+    torch.view_as_real refuses both."""
+    return t.data_ptr() if t.is_complex() and not t.is_conj() else torch.view_as_real(t).data_ptr()
 
 
 # The raw handle of a device's current stream: 0.06 us, where building a

@@ -6,6 +6,7 @@ import os
 import re
 
 import pytest
+import torch
 
 from qwen_image_accel import _native
 
@@ -208,3 +209,13 @@ def test_attention_workspace_bytes():
     for b, s, t, h in [(1, 300, 300, 2), (2, 520, 1500, 3), (1, 8, 20000, 1), (3, 700, 4352, 40)]:
         n = lib.qim_attention_workspace_bytes(b, s, t, h, 128)
         assert n >= vt(b, t, h) and (n - vt(b, t, h)) % part == 0
+
+
+def test_complex_ptr_refuses_what_holds_no_pairs():
+    """The RoPE table's address: a real or lazily conjugated table is refused,
+    as torch.view_as_real refuses it."""
+    table = torch.zeros(4, 2, dtype=torch.complex64)
+    assert _native.complex_ptr(table) == torch.view_as_real(table).data_ptr()
+    for bad in (torch.zeros(4, 4), torch.zeros(4, 2), table.conj()):
+        with pytest.raises(RuntimeError):
+            _native.complex_ptr(bad)

@@ -314,7 +314,8 @@ struct AttTile {
     uint32_t w[8];
     float e[2];     // P of a pair not yet packed
     float m;        // reference max (log2 units)
-    f32x4a_t l;     // this lane's sum of P (of the bf16 values used), in every element
+    float l;        // this lane's sum of P (of the bf16 values used), sub-blocks before the last one's
+    f32x4a_t r;     // the last sub-block's sum, in every element: added to l by att_sum
 };
 __device__ __forceinline__ bf16x8_t att_p(const AttTile &t, int u) {
     const u32x4_t v = {t.w[4 * u], t.w[4 * u + 1], t.w[4 * u + 2], t.w[4 * u + 3]};
@@ -324,10 +325,13 @@ __device__ __forceinline__ bf16x8_t att_p(const AttTile &t, int u) {
 // P = 2^(s c - m) of score k of a tile (called for k = 0..17 in order): the
 // exponential of score k, and for even k the packing of the pair before it (one
 // slot later, so that nothing waits for an exponential).  One slot after every
-// second pair its and the previous pair's four values are added to l: v_mfma_f32_4x4x4_16b_bf16 with an
+// second pair its and the previous pair's four values are added to r: v_mfma_f32_4x4x4_16b_bf16 with an
 // all-ones A is, for each lane, the sum of the lane's own four B values.  (As
 // v_dot2c_f32_bf16, eight per 16 scores, the sums slowed the MFMAs beside them:
-// 49.4 against 37.4 cycles per MFMA without them, loads left out.)
+// 49.4 against 37.4 cycles per MFMA without them, loads left out.)  r starts at
+// zero with each sub-block and is added to l once: 16 values whose exponents
+// differ by at most 12 add up exactly, and l, which grows with the keys, is
+// rounded once per 16 of them.
 __device__ __forceinline__ void att_exp(AttTile &t, int k, float c, i16x4_t ones) {
     if (k > 0 && k <= 16 && (k & 1) == 0) {
         uint32_t w = pack_bf16x2(t.e[0], t.e[1]);
@@ -337,10 +341,13 @@ __device__ __forceinline__ void att_exp(AttTile &t, int k, float c, i16x4_t ones
     }
     if (k > 4 && (k & 3) == 1) {
         const u32x2_t v = {t.w[(k - 1) / 2 - 2], t.w[(k - 1) / 2 - 1]};
-        t.l = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(i16x4_t, v), t.l, 0, 0, 0);
+        t.r = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(i16x4_t, v), k == 5 ? f32x4a_t{} : t.r, 0, 0,
+                                                     0);
     }
     if (k < 16) t.e[k & 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(t.s[k], c, -t.m));
 }
+
+__device__ __forceinline__ void att_sum(AttTile &t) { t.l += t.r[0]; }
 
 // Online softmax with a running max (the safe form).  Scores above the
 // reference max m by at most ATT_RESCALE (log2 units) are exponentiated
@@ -357,6 +364,7 @@ __device__ __forceinline__ void att_softmax_safe(AttTile &t, float c, i16x4_t on
     t.l *= alpha;
 #pragma unroll
     for (int k = 0; k <= 17; ++k) att_exp(t, k, c, ones);
+    att_sum(t);
     if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) t.o[dt] *= alpha;
@@ -384,8 +392,10 @@ __device__ __forceinline__ void att_wait_lds() {
 // MFMAs, and waited for each fragment separately.)  `work(k)` is the slot's memory
 // work.  LDSK: the fragments were read in the previous region, K first; at most
 // LDSK reads (V's) may be outstanding at the first score, none at the first P V.
-// FAST: B's reference max is fixed, nothing to rescale; otherwise the safe
-// softmax runs whole, before the MFMAs.
+// FAST: B's reference max is fixed, nothing to rescale; its sum r is complete
+// only at the region's end and is added to l in the next one (where the tile is
+// A), so that nothing waits for it.  Otherwise the safe softmax runs whole,
+// before the MFMAs.
 template <bool FAST, bool SCORES, bool PV, bool SOFTMAX, int LDSK, class F>
 __device__ __forceinline__ void att_region(AttTile &A, AttTile &B, const bf16x8_t (&q)[8], const bf16x8_t (&kf)[8],
                                            bf16x8_t (&vf)[2][4], float c, i16x4_t ones, F &&work) {
@@ -405,6 +415,8 @@ __device__ __forceinline__ void att_region(AttTile &A, AttTile &B, const bf16x8_
         }
         if (FAST) ATT_SCHED();
         if constexpr (FAST && SOFTMAX) att_exp(B, k, c, ones);
+        if constexpr (FAST && PV)
+            if (k == 2) att_sum(A);
         work(k);
         if (LDSK >= 0 && PV && k == 7) {
             att_wait_lds<0>();
@@ -454,7 +466,7 @@ __device__ __forceinline__ void att_pass(const AttnArgs &p, AttLoader ld, uint8_
     AttAddr A = att_addr<VT>(lane);
     bf16x8_t kf[8], vf[2][4];
     t0.m = t1.m = -__builtin_inff();
-    t0.l = t1.l = f32x4a_t{};
+    t0.l = t1.l = 0.f;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) t0.o[dt] = t1.o[dt] = f32x16a_t{};
 
@@ -604,7 +616,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
     AttTile t0, t1;
     att_pass<true, VT>(p, ld, lds, qf, wave, lane, kb0, nkb, t0, t1);
-    float l0 = t0.l[0], l1 = t1.l[0];
+    float l0 = t0.l, l1 = t1.l;
     // Rerun the whole workgroup in the safe form when any wave's sums left
     // the range the fixed reference max guarantees (scores that grew by more
     // than ~64 in log2 units past their first sub-block's max).
@@ -617,8 +629,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     if (__builtin_amdgcn_readfirstlane(redo[0] | redo[1] | redo[2] | redo[3])) {
         __syncthreads();  // read by every wave before the rings are filled again
         att_pass<false, VT>(p, att_start<VT>(p, b, h, kb0, nkb, wave, lane), lds, qf, wave, lane, kb0, nkb, t0, t1);
-        l0 = t0.l[0];
-        l1 = t1.l[0];
+        l0 = t0.l;
+        l1 = t1.l;
     }
 
     // O = O^T / l: lane (q, hf) holds dims 32dt + 8(i/4) + 4hf + i%4 of its query.

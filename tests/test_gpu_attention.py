@@ -176,3 +176,26 @@ def test_attention_output_stride_of_four(dev):
         out = wide[:, :, :384].unflatten(-1, (3, 128))
         attention.attention(q, k, v, out=out)
         assert torch.equal(out, want) and not wide[:, :, 384:].any()
+
+
+@pytest.mark.parametrize("s", [256, 8448])
+@pytest.mark.parametrize("redo", [False, True])
+def test_attention_row_sum_rounds_once_per_sub_block(dev, s, redo):
+    """The row sum's order: a lane's 16 keys of a sub-block are summed from zero
+    and added to its running sum once.  Every lane's sum is 16 after the first 32
+    keys (P = 1); each later sub-block brings 16 x 2^-23, one unit in the last
+    place of 16, of which any 4 are half lost.  V makes the first keys' mean
+    the midpoint 1 + 3 * 2^-8 of two bf16 values, so the 28 units tell on the
+    output: 1 + 2^-7, and the tie's 1 + 2^-6 without them.  960 keys (no split
+    over key ranges), V as rows and as tiles (more than 8192 queries), in the
+    first pass and in the redo (one query of the workgroup overflows it)."""
+    say("attention row sum", s, redo)
+    t = 960
+    q, k, v = (torch.zeros(1, n, 1, 128, dtype=torch.bfloat16) for n in (s, t, t))
+    q[..., 0], k[:, 32:, :, 0] = 1.0, -23.0
+    if redo:
+        q[:, 255, :, 0], q[:, 255, :, 1], k[:, 100, :, 1] = 0.0, 8.0, 64.0
+    v[:, 0:16], v[:, 16:32] = 1 + 2.0 ** -7, 1 + 2.0 ** -6
+    out = attention.attention(q.to(dev), k.to(dev), v.to(dev), scale=0.6931471805599453)
+    rows = [i for i in range(s) if not (redo and i == 255)]
+    assert (out.cpu()[:, rows] == 1 + 2.0 ** -7).all()

@@ -137,8 +137,17 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream(device=None):
-    """The current torch stream of `device` as a hipStream_t."""
-    index = None if device is None else torch.device(device).index
+    """The current torch stream of `device` as a hipStream_t.
+
+    Refuses a device that is no GPU, as torch.cuda.current_stream does: for
+    several wrappers it is the check that keeps a host tensor's address from
+    being launched with."""
+    index = None
+    if device is not None:
+        device = torch.device(device)
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        index = device.index
     if _raw_stream is None:
         return torch.cuda.current_stream(device).cuda_stream
     return _raw_stream(torch.cuda.current_device() if index is None else index)

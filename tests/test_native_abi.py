@@ -219,3 +219,70 @@ def test_complex_ptr_refuses_what_holds_no_pairs():
     for bad in (torch.zeros(4, 4), torch.zeros(4, 2), table.conj()):
         with pytest.raises(RuntimeError):
             _native.complex_ptr(bad)
+
+
+@pytest.fixture
+def one_gpu_seen(monkeypatch):
+    """The device queries of a process that has a GPU, and a recorder for native calls."""
+    launched = []
+    monkeypatch.setattr(_native, "call", lambda name, *args: launched.append(name))
+    monkeypatch.setattr(_native, "_raw_stream", lambda index: 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    return launched
+
+
+def _rope_qk(x, w, f):
+    from qwen_image_accel.kernels.elementwise import rope_qk
+    rope_qk(x, x, f)
+
+
+def _rms_norm(x, w, f):
+    from qwen_image_accel.kernels.bf16 import rms_norm
+    rms_norm(x, w, 1e-6)
+
+
+def _qk_norm_rope(x, w, f):
+    from qwen_image_accel.kernels.attention import qk_norm_rope
+    qk_norm_rope(x, x, w, w, f)
+
+
+def _host_quantized(rows, k):
+    from qwen_image_accel.kernels import mxfp8
+    return mxfp8.empty_quantized(rows, k, "cpu", tiled=True)
+
+
+def _mx_matmul(x, w, f):
+    from qwen_image_accel.kernels import gemm
+    q = _host_quantized(256, 128)
+    gemm.mx_matmul(_host_quantized(4, 128), q.values, q.scales, weight_tiled=True)
+
+
+def _mx_matmul_qk_norm_rope(x, w, f):
+    from qwen_image_accel.kernels import gemm
+    q = _host_quantized(768, 128)
+    gemm.mx_matmul_qk_norm_rope(_host_quantized(4, 128), q.values, q.scales, w, w, f, 2, 4, weight_tiled=True)
+
+
+def _linear_matmul(x, w, f):
+    from qwen_image_accel.optimizations.mxfp8 import MXFP8Linear
+    q = _host_quantized(256, 128)
+    MXFP8Linear.from_quantized(128, 256, q.values, q.scales).matmul(_host_quantized(4, 128))
+
+
+@pytest.mark.parametrize("entry", [_rope_qk, _rms_norm, _qk_norm_rope, _mx_matmul, _mx_matmul_qk_norm_rope,
+                                   _linear_matmul])
+def test_host_tensors_never_reach_a_launch(one_gpu_seen, entry):
+    """The wrappers that check no device themselves refuse host tensors when
+    they ask for the stream."""
+    x = torch.zeros(1, 4, 2, 128, dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        entry(x, torch.ones(128, dtype=torch.bfloat16), torch.zeros(4, 64, dtype=torch.complex64))
+    assert one_gpu_seen == []
+
+
+def test_stream_takes_gpus_only(one_gpu_seen):
+    for device in (None, "cuda", "cuda:0", torch.device("cuda", 1)):
+        assert _native.stream(device) == 0
+    for device in ("cpu", "cpu:0", "meta", torch.device("cpu")):
+        with pytest.raises(ValueError):
+            _native.stream(device)

@@ -286,3 +286,17 @@ def test_stream_takes_gpus_only(one_gpu_seen):
     for device in ("cpu", "cpu:0", "meta", torch.device("cpu")):
         with pytest.raises(ValueError):
             _native.stream(device)
+
+
+def test_attention_workspace_takes_gpus_only(monkeypatch, one_gpu_seen):
+    """A workspace's address is launched with, so no host buffer is one."""
+    from qwen_image_accel.kernels import attention
+    made, empty = [], torch.empty
+    monkeypatch.setattr(torch, "empty", lambda n, device, dtype: made.append(device) or empty(n, dtype=dtype))
+    for device in ("cpu", "meta", torch.device("cpu")):
+        with pytest.raises(ValueError):
+            attention.workspace(1, 64, 64, 1, device)
+    assert made == []
+    for device in ("cuda", "cuda:0", torch.device("cuda", 0)):
+        assert attention.workspace(1, 64, 64, 1, device).numel() == 16384
+    assert made == [torch.device("cuda"), torch.device("cuda", 0), torch.device("cuda", 0)]

@@ -81,7 +81,7 @@ SIGNATURES = {
 }
 
 _lib = None
-_functions = {}  # entry point name -> ctypes function, filled by lib()
+_functions = {}  # entry point name -> ctypes function; all of them once lib() has succeeded, none before
 _lock = threading.Lock()
 calls = {}  # entry point name -> number of successful launches (tests use it)
 
@@ -91,7 +91,7 @@ def available():
 
 
 def lib():
-    global _lib
+    global _lib, _functions
     if _lib is None:
         with _lock:
             if _lib is None:
@@ -99,12 +99,13 @@ def lib():
                     raise NativeUnavailable(
                         f"{LIB_PATH} is not built; run qwen-image-2.1-accel_amd/build_native.py")
                 handle = ctypes.CDLL(LIB_PATH, mode=ctypes.RTLD_LOCAL)
+                functions = {}
                 for name, (res, args) in SIGNATURES.items():
                     fn = getattr(handle, name)
                     fn.restype = res
                     fn.argtypes = args
-                    _functions[name] = fn
-                _lib = handle
+                    functions[name] = fn
+                _lib, _functions = handle, functions
     return _lib
 
 

@@ -300,3 +300,13 @@ def test_attention_workspace_takes_gpus_only(monkeypatch, one_gpu_seen):
     for device in ("cuda", "cuda:0", torch.device("cuda", 0)):
         assert attention.workspace(1, 64, 64, 1, device).numel() == 16384
     assert made == [torch.device("cuda"), torch.device("cuda", 0), torch.device("cuda", 0)]
+
+
+def test_library_that_lacks_a_symbol_is_refused_by_every_call(monkeypatch):
+    """A stale library: no call goes through, also not to the entry points it has."""
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(_native, "_functions", {})
+    monkeypatch.setattr(_native, "SIGNATURES", {**_native.SIGNATURES, "qim_no_such_entry": (ctypes.c_int, [])})
+    for _ in range(2):
+        with pytest.raises(AttributeError):
+            _native.call("qim_attention_workspace_bytes", 0, 0, 0, 0, 0)  # 0, which reads as QIM_OK

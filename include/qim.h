@@ -157,7 +157,8 @@ int qim_qk_norm_rope_pack(const void *q, const void *k, const void *v, const voi
  * bytes) + bs (swizzled over N rows).  fp32 accumulation.  Rows [0, M) are
  * written.  out: bf16 (M, Nout) with row stride ldo, Nout = N (N/2 for the
  * SWIGLU epilogues), or, for QIM_EPI_SWIGLU_QUANT, E4M3 codes (Mp, N/2) with
- * out_scales (Mp*N/64 bytes, swizzled).  bias: (N,) bf16.  gate: (B, N) bf16,
+ * out_scales (Mp*N/64 bytes, swizzled).  bias: (N,) bf16, any
+ * element address.  gate: (B, N) bf16,
  * res: (M, N) bf16 (row stride N), B = ceil(M / seq).
  * K % 128 == 0, N % 128 == 0 (the reference converts a linear when K and N
  * are multiples of 128, optimizations/mxfp8.py:15-16), N % 512 == 0 for the

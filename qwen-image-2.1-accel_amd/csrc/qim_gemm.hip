@@ -1323,6 +1323,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // lane per 8 columns of a row (16 lanes per row of a quarter, 16 rows per
 // workgroup), so that a few rows still spread over many waves; a lane's loads of
 // four partials are in flight together.
+// (The bias may start at any element: a slice of a larger buffer.)
+typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+
 template <int EPI>
 __global__ __launch_bounds__(256) void k_mx_gemm_sum(GemmArgs p) {
     static_assert(ring_offset<EPI>() == 0, "the split runs the plain, bias and gated-residual epilogues");
@@ -1336,7 +1339,8 @@ __global__ __launch_bounds__(256) void k_mx_gemm_sum(GemmArgs p) {
         hv = ld_nt(p.res + row * p.N + col);
         gv = *reinterpret_cast<const uint4 *>(p.gate + ((uint32_t)row / (uint32_t)p.seq) * p.N + col);
     } else if constexpr (EPI == QIM_EPI_BIAS) {
-        gv = *reinterpret_cast<const uint4 *>(p.bias + col);
+        const u32x4_any_t b = *reinterpret_cast<const u32x4_any_t *>(p.bias + col);
+        gv = make_uint4(b.x, b.y, b.z, b.w);
     }
     const float4 *w = reinterpret_cast<const float4 *>(p.ws + (int64_t)q * QPART_WORDS + r * 128 + c);
     const int64_t step = (int64_t)p.quarters * (QPART_WORDS / 4);

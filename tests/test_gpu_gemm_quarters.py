@@ -90,3 +90,20 @@ def test_swiglu_quarter_grid(dev, m, f, k):
         got = gemm.mx_matmul(x, q.values, q.scales, epilogue="swiglu_quant", weight_tiled=True, out_tiled=tiled)
         ref = mxfp8.quantize(want, tiled=tiled)
         assert np.array_equal(u8(got.values), u8(ref.values)) and np.array_equal(u8(got.scales), u8(ref.scales))
+
+
+# A grid of quarter tiles split over K, and whole tiles whose tail is split (272 tiles).
+@pytest.mark.parametrize("m,n,k", [(40, 4096, 4096), (4352, 4096, 1024)])
+def test_split_bias_at_any_element(dev, m, n, k):
+    """The bias of a split grid may be a slice that starts at any element."""
+    assert _native.lib().qim_mxfp8_gemm_ws_bytes(m, n, k, _native.EPI_BIAS) > 0
+    print("[case] split, bias at any element", m, n, k, flush=True)
+    g = torch.Generator().manual_seed(m + n)
+    a, w = bf16_randn(g, (m, k)).to(dev), bf16_randn(g, (n, k), 0.05).to(dev)
+    aq, wq = mxfp8.quantize(a), mxfp8.quantize(w)
+    buf = bf16_randn(g, (n + 8,)).to(dev)
+    y32 = gemm.mx_matmul(aq, wq.values, wq.scales, dtype=torch.float32)
+    for at in (0, 1, 2, 5, 7):
+        bias = buf[at:at + n]
+        y = gemm.mx_matmul(aq, wq.values, wq.scales, epilogue="bias", bias=bias)
+        assert torch.equal(y, (y32 + bias.float()).to(torch.bfloat16)), at

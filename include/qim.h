@@ -253,7 +253,7 @@ int qim_mxfp8_gemm_qk_norm_rope_vt(const void *aq, const void *as, const void *b
  * the partial results of work items split over key ranges to fill the last
  * round of workgroups; the split depends on the current device's CU count).
  * v = NULL (ldv ignored): the workspace already holds V^T, written by
- * qim_mxfp8_gemm_qk_norm_rope_vt; T % 64 == 0. */
+ * qim_mxfp8_gemm_qk_norm_rope_vt; T % 64 == 0.  The output may lie over v. */
 int qim_attention(const void *q, int64_t ldq, const void *k, int64_t ldk, const void *v, int64_t ldv,
                   void *o, int64_t ldo, void *workspace, int64_t workspace_bytes, int64_t B, int64_t S,
                   int64_t T, int64_t H, int64_t D, float scale, void *stream);

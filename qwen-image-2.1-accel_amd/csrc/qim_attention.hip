@@ -832,6 +832,11 @@ AttPlan att_plan(int64_t B, int64_t S, int64_t T, int64_t H) {
     return pl;
 }
 
+static bool ranges_overlap(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + (uintptr_t)b_bytes && y < x + (uintptr_t)a_bytes;
+}
+
 // The checks and launches the attention entry points share.  Output: bf16 rows
 // of o (ldo elements apart), or MXFP8 codes and scales when qcodes is set.
 // v null: the workspace already holds V^T (qim_mxfp8_gemm_qk_norm_rope_vt),
@@ -862,8 +867,16 @@ int attention_run(const char *who, const void *q, int64_t ldq, const void *k, in
                 "%s: workspace of %lld bytes, this problem needs %lld (qim_attention_workspace_bytes)", who,
                 (long long)workspace_bytes, (long long)pl.total());
     // V rows read through the transposing LDS reads, or V^T tiles: from the
-    // workspace when v is null, else made here.
-    const bool vt = !v || S > ATT_VROWS_MAX_S || ldv >= (1ll << 25);  // (32-bit row offsets)
+    // workspace when v is null, else made here.  V rows are read until the last
+    // workgroup ends, so an output whose memory overlaps V's takes V^T tiles,
+    // which are complete before the first output is written.
+    const int64_t M = B * S, Mp = (M + 127) / 128 * 128;
+    bool vt = !v || S > ATT_VROWS_MAX_S || ldv >= (1ll << 25);  // (32-bit row offsets)
+    if (!vt) {
+        const int64_t v_bytes = ((B * T - 1) * ldv + H * D) * 2;
+        vt = qcodes ? ranges_overlap(v, v_bytes, qcodes, Mp * H * D) || ranges_overlap(v, v_bytes, qscales, Mp * H * D / 32)
+                    : ranges_overlap(v, v_bytes, o, ((M - 1) * ldo + H * D) * 2);
+    }
     static std::atomic<bool> configured[4][QIM_MAX_DEVICES] = {};
     void (*const fwd)(AttnArgs) = qcodes ? (vt ? k_attn_fwd<true, true> : k_attn_fwd<true, false>)
                                          : (vt ? k_attn_fwd<false, true> : k_attn_fwd<false, false>);
@@ -896,10 +909,9 @@ int attention_run(const char *who, const void *q, int64_t ldq, const void *k, in
     a.part_o = reinterpret_cast<uint16_t *>(ws + pl.vt_bytes);
     a.part_ml = reinterpret_cast<float *>(ws + pl.vt_bytes + pl.part_o_bytes);
     a.scale_log2e = scale * 1.4426950408889634f;
-    const int64_t M = B * S;
     a.qcodes = static_cast<uint8_t *>(qcodes);
     a.qscales = static_cast<uint8_t *>(qscales);
-    a.Mp = (M + 127) / 128 * 128;
+    a.Mp = Mp;
     a.tiled = tiled;
     a.o_vec16 = o && aligned16(o) && ldo % 8 == 0;
     const int64_t nwg = pl.nfull + pl.ntail * pl.nsplit;

@@ -199,3 +199,29 @@ def test_attention_row_sum_rounds_once_per_sub_block(dev, s, redo):
     out = attention.attention(q.to(dev), k.to(dev), v.to(dev), scale=0.6931471805599453)
     rows = [i for i in range(s) if not (redo and i == 255)]
     assert (out.cpu()[:, rows] == 1 + 2.0 ** -7).all()
+
+
+@pytest.mark.parametrize("t", [520, 1500])
+def test_attention_output_over_v(dev, t):
+    """The output may lie over V (whole items, and items split over key ranges
+    and merged): as bf16 rows, as rows of a fused QKV buffer, and as MXFP8 codes."""
+    b, h = 2, 3
+    say("attention output over v", t)
+    g = torch.Generator().manual_seed(t)
+    qkv = bf16_randn(g, (b, t, 3 * h * 128)).to(dev)
+    q, k, v = (qkv[:, :, i * h * 128:(i + 1) * h * 128].unflatten(-1, (h, 128)) for i in range(3))
+    want = attention.attention(q, k, v).clone()
+    ref = mxfp8.quantize(want.view(b * t, h * 128), tiled=True)
+    over = v.contiguous()
+    assert torch.equal(attention.attention(q, k, over, out=over), want)
+    # Codes in V's own memory (a V with rows to spare for the padded code rows).
+    buf = torch.empty(ref.values.numel(), device=dev, dtype=torch.bfloat16)
+    over = buf[:b * t * h * 128].view(b, t, h, 128)
+    over.copy_(v)
+    out = ref._replace(values=buf.view(torch.uint8)[:ref.values.numel()].view(ref.values.dtype).view(ref.values.shape),
+                       scales=torch.empty_like(ref.scales))
+    attention.attention_mxfp8(q, k, over, out=out)
+    assert torch.equal(out.values.view(torch.uint8), ref.values.view(torch.uint8))
+    assert torch.equal(out.scales.view(torch.uint8), ref.scales.view(torch.uint8))
+    attention.attention(q, k, v, out=v)
+    assert torch.equal(v, want)

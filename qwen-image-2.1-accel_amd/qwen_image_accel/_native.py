@@ -145,7 +145,8 @@ def stream(device=None):
     being launched with."""
     index = None
     if device is not None:
-        device = torch.device(device)
+        if not isinstance(device, torch.device):
+            device = torch.device(device)
         if device.type != "cuda":
             raise ValueError(f"Expected a cuda device, but got: {device}")
         index = device.index

@@ -83,16 +83,18 @@ def test_attention_on_fused_qkv_views(dev):
     check(out, reference(q, k, v, 0.1))
 
 
+# 256 queries read V as rows, 8448 as V^T tiles.
+@pytest.mark.parametrize("s", [256, 8448])
 @pytest.mark.parametrize("jump", [30.0, 400.0])
-def test_attention_score_jump_past_first_block(dev, jump):
+def test_attention_score_jump_past_first_block(dev, jump, s):
     """Keys whose scores exceed the scores of the first 32 keys by about
     `jump` (natural-log units).  The kernel's first pass keeps each query's
     reference max from its first key sub-block: a jump of 30 stays within
     its range (P up to ~e^33, l and O finite), one of 400 overflows it, which
     the kernel detects and redoes in the running-max form.  Either way the
-    output equals the reference."""
-    b, s, t, h = 1, 256, 700, 2
-    say("attention score jump", jump)
+    output equals the reference, and the MXFP8 form its quantization."""
+    b, t, h = 1, 700, 2
+    say("attention score jump", jump, s)
     g = torch.Generator().manual_seed(int(jump))
     # Head 0: every query is q0 plus a little noise; keys 600..609 are q0
     # scaled to a logit of about `jump` against it.
@@ -108,6 +110,28 @@ def test_attention_score_jump_past_first_block(dev, jump):
     ref = reference(q, k, v, scale)
     assert torch.isfinite(out.float()).all()
     check(out, ref)
+    got, want = attention.attention_mxfp8(q, k, v, tiled=False), mxfp8.quantize(out.view(s, h * 128))
+    assert torch.equal(got.values.view(torch.uint8), want.values.view(torch.uint8))
+    assert torch.equal(got.scales.view(torch.uint8), want.scales.view(torch.uint8))
+    if s > 256:  # 700 keys are too few to split: the first queries' workgroups, with V as rows
+        rows = attention.attention(q[0, :256].unsqueeze(0), k, v)
+        assert torch.equal(out[:, :256].contiguous().view(torch.int16), rows.view(torch.int16))
+
+
+def test_attention_v_tiles_split_ragged(dev):
+    """V^T tiles (more than 8192 queries) with the items split over key ranges
+    and a last key block of 28 keys."""
+    from qwen_image_accel import _native
+    b, s, t, h = 1, 8448, 1500, 2
+    say("attention v tiles, split, ragged", s, t)
+    assert _native.lib().qim_attention_workspace_bytes(b, s, t, h, 128) > b * h * 24 * 16384  # V^T and partials
+    g = torch.Generator().manual_seed(t)
+    q, k, v = (bf16_randn(g, (b, n, h, 128)).to(dev) for n in (s, t, t))
+    out = attention.attention(q, k, v)
+    check(out, reference(q, k, v, 128 ** -0.5))
+    got, want = attention.attention_mxfp8(q, k, v, tiled=True), mxfp8.quantize(out.view(s, h * 128), tiled=True)
+    assert torch.equal(got.values.view(torch.uint8), want.values.view(torch.uint8))
+    assert torch.equal(got.scales.view(torch.uint8), want.scales.view(torch.uint8))
 
 
 # (2, 200, 333, 3): 400 rows, padded to 512, past the last query block's end;

@@ -2,7 +2,9 @@
 CU), unsplit and split over K through a workspace, at the edges of that range:
 one row, one stage pair of K, a K whose pairs do not divide into the splits,
 rows that leave dead 32-row groups, one more row than a quarter tile, and the
-largest grid (512 quarter tiles on 256 CUs) with its first whole-tile neighbour.
+largest grid (512 quarter tiles on 256 CUs) with its neighbour of one more row
+(which runs as 192 x 256 tiles).  And grids of 256 x 256 tiles, at the smallest K
+of their ring, with the quarter tiles of their last partial round.
 """
 import numpy as np
 import pytest
@@ -107,3 +109,70 @@ def test_split_bias_at_any_element(dev, m, n, k):
         bias = buf[at:at + n]
         y = gemm.mx_matmul(aq, wq.values, wq.scales, epilogue="bias", bias=bias)
         assert torch.equal(y, (y32 + bias.float()).to(torch.bfloat16)), at
+
+
+@pytest.mark.parametrize("k", [128, 384])
+def test_mxfp8_gemm_whole_tile_grid(dev, k):
+    """4352 x 4096: 256 whole tiles, then 64 quarter tiles (split over K at K =
+    384), at one and three stage pairs, in every output format, against the
+    oracle and the same rows as unsplit quarter tiles (bit for bit, but for the
+    rows of the split tail)."""
+    m, n = 4352, 4096
+    ws = _native.lib().qim_mxfp8_gemm_ws_bytes(m, n, k, _native.EPI_NONE)
+    print("[case] whole tiles", m, n, k, "workspace", ws, flush=True)
+    assert (ws > 0) == (k > 128)
+    g = torch.Generator().manual_seed(k)
+    a, w, bias = bf16_randn(g, (m, k)).to(dev), bf16_randn(g, (n, k), 0.05).to(dev), bf16_randn(g, (n,)).to(dev)
+    aq, wq = mxfp8.quantize(a), mxfp8.quantize(w)
+    at, wt = mxfp8.quantize(a, tiled=True), mxfp8.quantize(w, tiled=True)
+
+    def unsplit(x, out, flag):
+        _native.call("qim_mxfp8_gemm_ex", _native.ptr(x.values), _native.ptr(x.scales), _native.ptr(wq.values),
+                     _native.ptr(wq.scales), x.rows, n, k, _native.EPI_NONE, flag, None, None, None, x.rows,
+                     _native.ptr(out), n, None, _native.stream(dev))
+        return out
+    u32 = unsplit(aq, torch.empty(m, n, device=dev, dtype=torch.float32), _native.GEMM_OUT_F32)
+    rows = np.unique(np.concatenate([np.arange(24), np.arange(m - 24, m), np.arange(0, m, 193)]))
+    ref = O.mx_gemm(u8(aq.values), u8(aq.scales), u8(wq.values), u8(wq.scales), rows=rows)
+    assert rel_fro(u32.cpu().numpy()[rows], ref) < 1e-2
+    for r0 in range(0, m, 512):
+        x = mxfp8.quantize(a[r0:r0 + 512])
+        part = unsplit(x, torch.empty(x.rows, n, device=dev, dtype=torch.float32), _native.GEMM_OUT_F32)
+        assert torch.equal(part, u32[r0:r0 + 512]), r0
+    assert torch.equal(unsplit(aq, torch.empty(m, n, device=dev, dtype=torch.float16), _native.GEMM_OUT_F16),
+                       u32.to(torch.float16))
+    assert torch.equal(unsplit(aq, torch.empty(m, n, device=dev, dtype=torch.bfloat16), 0), u32.to(torch.bfloat16))
+    # Through the workspace (the tail's rows: fp32 sums of the same products in another order).
+    y32 = gemm.mx_matmul(aq, wq.values, wq.scales, dtype=torch.float32)
+    assert (y32 - u32).abs().max().item() <= 1e-5 * u32.abs().max().item()
+    assert torch.equal(gemm.mx_matmul(aq, wq.values, wq.scales, dtype=torch.float16), y32.to(torch.float16))
+    for x, ww, tiled in ((aq, wq, False), (at, wq, False), (aq, wt, True), (at, wt, True)):
+        y = gemm.mx_matmul(x, ww.values, ww.scales, epilogue="bias", bias=bias, weight_tiled=tiled)
+        assert torch.equal(y, (y32 + bias.float()).to(torch.bfloat16))
+
+
+def test_swiglu_whole_tile_grid(dev):
+    """The SwiGLU epilogues of whole tiles (silu looked up) and of the tail's
+    quarter tiles, with gate values outside the table's range and zeros, against
+    the unfused GEMM, swiglu and quantizer, byte for byte."""
+    from qwen_image_accel.kernels.bf16 import swiglu
+    m, f, k = 4352, 2048, 128
+    print("[case] swiglu whole tiles", m, f, k, flush=True)
+    g = torch.Generator().manual_seed(m)
+    a = bf16_randn(g, (m, k))
+    a[::7] *= 64
+    wg, wu = bf16_randn(g, (f, k), 0.2), bf16_randn(g, (f, k), 0.2).to(dev)
+    wg[::5] = 0
+    wg = wg.to(dev)
+    x = mxfp8.quantize(a.to(dev), tiled=True)
+    q = mxfp8.quantize(gemm.interleave_swiglu(wg, wu), tiled=True)
+    assert _native.lib().qim_mxfp8_gemm_ws_bytes(m, f, k, _native.EPI_NONE) == 0  # the sums below are unsplit
+    gate, up = (gemm.mx_matmul(x, w.values, w.scales, weight_tiled=True)
+                for w in (mxfp8.quantize(wg, tiled=True), mxfp8.quantize(wu, tiled=True)))
+    assert gate.abs().max() > 100 and (gate[:, ::5] == 0).all() and (up[:, ::5] != 0).any()
+    want = swiglu(gate, up)
+    assert torch.equal(gemm.mx_matmul(x, q.values, q.scales, epilogue="swiglu", weight_tiled=True), want)
+    for tiled in (False, True):
+        got = gemm.mx_matmul(x, q.values, q.scales, epilogue="swiglu_quant", weight_tiled=True, out_tiled=tiled)
+        ref = mxfp8.quantize(want, tiled=tiled)
+        assert np.array_equal(u8(got.values), u8(ref.values)) and np.array_equal(u8(got.scales), u8(ref.scales))

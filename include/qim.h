@@ -249,8 +249,9 @@ int qim_mxfp8_gemm_qk_norm_rope_vt(const void *aq, const void *as, const void *b
  * tokens (views into a fused QKV output are fine).  D = 128, scale > 0.  fp32
  * scores, softmax and accumulation; P rounded to bf16 for the P V product.
  * workspace: at least qim_attention_workspace_bytes(B, S, T, H, D) bytes,
- * 16-byte aligned, passed with its size (V transposed in 64-key tiles, and
- * the partial results of work items split over key ranges to fill the last
+ * 16-byte aligned, passed with its size (room for V transposed in 64-key
+ * tiles, which is used above 8192 queries or where o overlaps v, and the
+ * partial results of work items split over key ranges to fill the last
  * round of workgroups; the split depends on the current device's CU count).
  * v = NULL (ldv ignored): the workspace already holds V^T, written by
  * qim_mxfp8_gemm_qk_norm_rope_vt; T % 64 == 0.  The output may lie over v. */

@@ -8,7 +8,8 @@ namespace qim {
 
 // How one attention problem is run: workgroups [0, nfull) run whole work
 // items, the ntail items after them run as nsplit chunks of kbc key blocks;
-// the workspace holds the V^T tiles (vt_bytes), then the chunks' bf16 output
+// the workspace holds room for the V^T tiles (vt_bytes; unused where V is read
+// as rows), then the chunks' bf16 output
 // rows (part_o_bytes) and fp32 (m, l) pairs (part_ml_bytes).
 struct AttPlan {
     int64_t nfull, ntail, nsplit, kbc;

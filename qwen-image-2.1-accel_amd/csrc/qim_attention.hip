@@ -26,11 +26,17 @@
 // (conflict-free reads of 16 lanes with consecutive d).  K is loaded straight from
 // the K tensor, with chunk c of key r at chunk c ^ (r & 15) in LDS.
 //
-// What bounds it: long runs draw the power limit (S = T = 16640, 24 heads: ~1.74
-// GHz, the matrix cores busy 71 % of the waves' cycles, 47.7 cycles per 32-cycle
-// MFMA; 58 with the row sums on v_dot2c_f32_bf16, 54 as the compiler scheduled
-// them).  S 16640 2950 -> 2850 us, S 4096 x T 8392 (32 heads) 588 -> 536 us, S 1024
-// x T 1101 (2 x 32 heads) 62 -> 44 us including the transpose pass this drops.
+// What bounds it: the clock, 1.84-1.87 GHz of 2.4 in long runs (power limit), and
+// the cycles beyond the matrix cores' own.  Counters, per 32-cycle MFMA of a wave:
+// S = T = 16640, 24 heads, V^T tiles 44.9 cycles, of which the matrix core is busy
+// 34.0 (2 for the row sums; 76 %); the wave issues in 25.2, has an instruction ready
+// that cannot issue in 13.0 and waits (barrier, LDS, loads) in 6.7.  S 4096 x T 8392,
+// 32 heads, V rows: 49.6, busy 34.0 (69 %), 28.3, 13.1 and 8.2.  No LDS bank
+// conflicts in either.  How much of the waits are barriers and how much are loads was
+// not separated.  Against the schedule the compiler made with every call
+// transposing V (same box each): S = T = 16640 2785 -> 2600 us, S 4096 x T 8392 496 ->
+// 443 us, S = T = 4352 (24 heads) 231 -> 208 us, S 1024 x T 1101 (2 x 32 heads) 54.7 ->
+// 40.5 us.
 #include <type_traits>
 
 #include "qim_attention.h"
@@ -387,7 +393,8 @@ __device__ __forceinline__ void att_wait_lds() {
 // slots of one MFMA and one score each.  A lone wave issues at most one
 // instruction per 4.4 cycles (5.4 for an 8-byte one, 8.5 for an exponential), so
 // a slot of one MFMA, a score's fma and exponential, half a pack and a row sum and
-// one LDS read just fits the MFMA's 32 cycles.  (Left to itself the compiler
+// one LDS read could fit the MFMA's 32 cycles; what the whole loop takes stands at
+// the head of the file.  (Left to itself the compiler
 // bunched the softmax into the first half of each region, left the rest to bare
 // MFMAs, and waited for each fragment separately.)  `work(k)` is the slot's memory
 // work.  LDSK: the fragments were read in the previous region, K first; at most
@@ -785,7 +792,7 @@ using namespace qim;
 // one fits per CU, so W whole items take ceil(W / CUs) rounds; when the last
 // round is partial, its items may run instead as chunks of kbc key blocks plus
 // a merge pass.  Cost model, in units of one workgroup's time per 64-key
-// block (measured ~1.75 us at 24 heads): whole rounds * nkb + chunk rounds *
+// block (1.75 us at 24 heads when the model was made, 1.6 now): whole rounds * nkb + chunk rounds *
 // kbc + the partials' HBM traffic (written once, read once by the merge, at
 // ~5 TB/s) + ~3 for the merge launch.  A split is taken when it saves >= 5 %;
 // chunks have at least ATT_MIN_CHUNK blocks.  Partials are bf16 rows and
@@ -797,9 +804,10 @@ namespace qim {
 constexpr int ATT_MIN_CHUNK = 8;
 // Most queries per image for which V is read as rows: the transposing reads
 // take two instructions per fragment, the transpose pass one trip of V through
-// memory, and the reads are repeated by every query block.  Rows against V^T:
-// S 1024, T 1101, B 2, H 32 49.9 / 59.6 us; S 4352 264 / 266 us; S 8192 797 / 790
-// us; S 16640 2889 / 2848 us.
+// memory, and the reads are repeated by every query block.  Rows against V^T with
+// its pass: S 1024, T 1101, B 2, H 32 42.7 / 52.9 us; S = T = 1280, H 24 32.3 / 37.7;
+// S 4096, T 8392, H 32 463 / 477; S = T = 4352, H 24 212 / 217; S = T = 8192, H 24 672.0
+// / 671.8, H 32 893.0 / 891.8; S = T = 16640, H 24 2765 / 2718 us.
 constexpr int64_t ATT_VROWS_MAX_S = 8192;
 
 AttPlan att_plan(int64_t B, int64_t S, int64_t T, int64_t H) {
@@ -840,7 +848,8 @@ static bool ranges_overlap(const void *a, int64_t a_bytes, const void *b, int64_
 // The checks and launches the attention entry points share.  Output: bf16 rows
 // of o (ldo elements apart), or MXFP8 codes and scales when qcodes is set.
 // v null: the workspace already holds V^T (qim_mxfp8_gemm_qk_norm_rope_vt),
-// T % 64 == 0.
+// T % 64 == 0.  The workspace always has the room for V^T, also where V is read as
+// rows: its size is asked for before it is known whether the output overlaps V.
 int attention_run(const char *who, const void *q, int64_t ldq, const void *k, int64_t ldk, const void *v,
                          int64_t ldv, void *o, int64_t ldo, void *qcodes, void *qscales, int tiled, void *workspace,
                          int64_t workspace_bytes, int64_t B, int64_t S, int64_t T, int64_t H, int64_t D, float scale,

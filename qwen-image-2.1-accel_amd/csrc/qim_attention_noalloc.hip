@@ -1,15 +1,15 @@
 // qim_attention_noalloc: the attention core with its workspace in a buffer the
 // library owns, for callers that cannot allocate device memory (code under HIP
-// graph capture, tight serving loops).  The workspace of qim_attention (the
-// V^T tiles, and the partial rows of work items split over key ranges) lives
+// graph capture, tight serving loops).  The workspace of qim_attention (room for
+// the V^T tiles, and the partial rows of work items split over key ranges) lives
 // in `scratch`, a file-scope device array of QIM_ATTENTION_NOALLOC_MAX_BYTES.
 // Each device holds its own copy from the first call on it until the process
 // ends; its address on each device is resolved once, with that device
 // current, and kept in g_scratch.  Every call on a device reuses the array, so
 // calls that overlap on one device race.  No call needs the array cleared:
-// every byte a call reads was written earlier in the same call (k_attn_vt
-// writes whole V^T tiles, zeros past the last key; each split chunk writes its
-// partial rows before the merge pass reads them).
+// every byte a call reads was written earlier in the same call (where V is read as
+// V^T tiles, k_attn_vt writes whole ones, zeros past the last key; each split chunk
+// writes its partial rows before the merge pass reads them).
 #include <mutex>
 
 #include "qim_attention.h"

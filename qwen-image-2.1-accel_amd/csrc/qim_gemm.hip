@@ -736,7 +736,8 @@ __device__ __forceinline__ void epilogue(const GemmArgs &p, f32x16_t (&acc)[TI][
                 // the other half is the partner wave's (wave ^ 1, same rows),
                 // whose row sums come through LDS.  The Q/K/V class is uniform
                 // over a quarter tile's four waves (one head), so its barriers
-                // are too.
+                // are too.  So it is over the four waves of a 192-row tile (two
+                // heads): H is even, so both heads are of one class.
                 if (qk_cols) {
                     float x[4][8];
                     double ss[4];
@@ -1509,7 +1510,11 @@ static GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, int epilogue) {
     // (quarters * ksplit <= CUs), at most one stage pair each and at most 8; 1
     // (no split) when the quarters alone hold more than half the CUs, when a last
     // 128-column block is there, or for an epilogue other than the plain, bias
-    // and gated-residual ones.
+    // and gated-residual ones.  Unlike quarter_ksplit this asks for no gain, and
+    // below about K 4096 there is none: unsplit / split (bias), 4352 x 4096: K 1024
+    // 24.2 / 28.3 us, 3072 49.6 / 50.4, 4096 62.7 / 61.9, 12288 164.7 / 153.5; 4608 x 4096
+    // (128 quarters in 2): K 4096 63.5 / 67.0, 12288 166.6 / 165.7; 16640 x 3072 (48
+    // in 5): K 3072 120.8 / 121.7, 12288 414.8 / 408.2 us.
     if (pl.quarters > 0 && tiles_n * BN == N && splits_k(epilogue)) {
         int64_t k = cus / pl.quarters;
         k = k < pairs ? k : pairs;

@@ -58,8 +58,8 @@ def prepare_attention_inputs(q, k, v, norm_q, norm_k, freqs, cached_k, cached_v)
 
 
 def workspace(b, s, t, h, device, d=128):
-    """A workspace for ``attention`` / ``attention_mxfp8`` of this shape (V^T
-    tiles first, then the split items' partial results)."""
+    """A workspace for ``attention`` / ``attention_mxfp8`` of this shape (room
+    for V^T tiles first, then the split items' partial results)."""
     device = torch.get_default_device() if device is None else torch.device(device)
     if device.type != "cuda":
         raise ValueError(f"Expected a cuda device, but got: {device}")

@@ -845,6 +845,14 @@ static bool ranges_overlap(const void *a, int64_t a_bytes, const void *b, int64_
     return x < y + (uintptr_t)b_bytes && y < x + (uintptr_t)a_bytes;
 }
 
+// Whether rows of `width` bytes, `stride` bytes apart, from a and from b are column
+// blocks of one buffer that share no column.
+static bool columns_disjoint(const void *a, const void *b, int64_t stride, int64_t width) {
+    const int64_t d = (int64_t)(reinterpret_cast<uintptr_t>(a) - reinterpret_cast<uintptr_t>(b));
+    const int64_t r = (d % stride + stride) % stride;  // a's first column seen from b's
+    return r >= width && r + width <= stride;
+}
+
 // The checks and launches the attention entry points share.  Output: bf16 rows
 // of o (ldo elements apart), or MXFP8 codes and scales when qcodes is set.
 // v null: the workspace already holds V^T (qim_mxfp8_gemm_qk_norm_rope_vt),
@@ -884,7 +892,8 @@ int attention_run(const char *who, const void *q, int64_t ldq, const void *k, in
     if (!vt) {
         const int64_t v_bytes = ((B * T - 1) * ldv + H * D) * 2;
         vt = qcodes ? ranges_overlap(v, v_bytes, qcodes, Mp * H * D) || ranges_overlap(v, v_bytes, qscales, Mp * H * D / 32)
-                    : ranges_overlap(v, v_bytes, o, ((M - 1) * ldo + H * D) * 2);
+                    : ranges_overlap(v, v_bytes, o, ((M - 1) * ldo + H * D) * 2) &&
+                          !(ldo == ldv && columns_disjoint(o, v, ldo * 2, H * D * 2));
     }
     static std::atomic<bool> configured[4][QIM_MAX_DEVICES] = {};
     void (*const fwd)(AttnArgs) = qcodes ? (vt ? k_attn_fwd<true, true> : k_attn_fwd<true, false>)

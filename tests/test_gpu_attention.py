@@ -247,5 +247,11 @@ def test_attention_output_over_v(dev, t):
     attention.attention_mxfp8(q, k, over, out=out)
     assert torch.equal(out.values.view(torch.uint8), ref.values.view(torch.uint8))
     assert torch.equal(out.scales.view(torch.uint8), ref.scales.view(torch.uint8))
-    attention.attention(q, k, v, out=v)
-    assert torch.equal(v, want)
+    # Column blocks of one buffer: beside V, over Q, across two heads of V, over V.
+    w = h * 128
+    for at in (3 * w, 0, 2 * w + 128, 2 * w):
+        wide = torch.zeros(b, t, 4 * w, device=dev, dtype=torch.bfloat16)
+        wide[:, :, :3 * w] = qkv
+        wq, wk, wv, o = (wide[:, :, c:c + w].unflatten(-1, (h, 128)) for c in (0, w, 2 * w, at))
+        attention.attention(wq, wk, wv, out=o)
+        assert torch.equal(o, want), at
